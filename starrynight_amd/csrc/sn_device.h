@@ -57,60 +57,148 @@ __device__ __forceinline__ void philox4x32_10(uint32_t c[4], uint32_t k0, uint32
     }
 }
 
+// The disc coordinate of a Philox word: x = a 2^-26, a odd, |a| < 2^26.
+__device__ __forceinline__ double disc_coordinate(uint32_t word)
+{
+    return (double)((int)((word >> 5) | 1u) - (1 << 26)) * (1.0 / 67108864.0);
+}
+
+// |x|^2 of a candidate: the squares have at most 52 bits and their sum fits in
+// 53, so nothing rounds.
+__device__ __forceinline__ double disc_norm2(double x1, double x2) { return fma(x1, x1, x2 * x2); }
+
+// sqrt of x in [2^-52, 1], correctly rounded: Goldschmidt iterations from the
+// hardware's reciprocal root and two residual corrections (Markstein).  The
+// library's sqrt spends as much again on scaling denormals and on zero and
+// infinity, none of which occur here.
+__device__ __forceinline__ double sqrt_unit(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+
+// ln u of u = j 2^-53, 0 < j < 2^53: u = 2^k m with m in [sqrt(1/2), sqrt 2),
+// ln m = 2 atanh(t), t = (m - 1) / (m + 1) carried in two doubles (m - 1 is
+// exact), atanh by its Taylor series (t^2 < 0.0295: eleven terms reach 2^-56),
+// k ln 2 in two doubles.  At most 0.56 ulp off (20 million arguments against
+// an extended-precision log); about 50 instructions against the library's 118,
+// most of them a dependent chain that a wave waits for.
+__device__ __forceinline__ double log_unit(double u)
+{
+    double m = __builtin_amdgcn_frexp_mant(u);   // [1/2, 1)
+    int k = __builtin_amdgcn_frexp_exp(u);
+    const bool low = m < 0.70710678118654752440;
+    m = low ? 2.0 * m : m;
+    k -= low ? 1 : 0;
+    const double f = m - 1.0, d = m + 1.0, de = (1.0 - d) + m;   // d + de = m + 1
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(fma(-d, r, 1.0), r, r);
+    r = fma(fma(-d, r, 1.0), r, r);
+    const double t = f * r, tl = fma(-de, t, fma(-d, t, f)) * r;   // t + tl = f / (m + 1)
+    const double z = t * t, z2 = z * z, z4 = z2 * z2;
+    const double a = fma(z2, fma(z, 1.0 / 9, 1.0 / 7), fma(z, 1.0 / 5, 1.0 / 3));
+    const double b = fma(z4, fma(z, 1.0 / 21, 1.0 / 19),
+                         fma(z2, fma(z, 1.0 / 17, 1.0 / 15), fma(z, 1.0 / 13, 1.0 / 11)));
+    const double lo = fma(t * z, fma(z4, b, a), tl);
+    const double kd = (double)k, h2 = 2.0 * t;
+    const double kh = kd * 0x1.62e42fefa3800p-1;   // exact: the constant's low 11 bits are zero
+    const double h = kh + h2;
+    const double e = k != 0 ? (kh - h) + h2 : 0.0;   // (|kh| > |h2|)
+    return h + (e + fma(kd, 0x1.ef35793c76730p-45, 2.0 * lo));
+}
+
 // Proposal and acceptance uniform for one visit of `site` in `sweep`:
 // counter (site, sweep, replica, k), key = seed.  u = 53-bit uniform from words
 // 2, 3 of k = 0; Marsaglia (1972) disc point from words 0, 1 of k = 0, then
 // words 0, 1 and 2, 3 of k = 1, 2, ... (two candidates per retry call: a
 // wave waits for its slowest lane, so fewer calls per rejection shorten every
-// draw), with x = a 2^-26, a odd: the disc test is exact in integers and
-// 1 - s, 1 - 2 s are exact, so only one sqrt and two products round.
-__device__ __forceinline__ void counter_draw(unsigned long long seed, uint32_t replica,
-                                             uint32_t sweep, uint32_t site, int constrain_to_x,
-                                             double &px, double &py, double &pz, double &u)
+// draw), with x = a 2^-26, a odd: the disc test and 1 - s, 1 - 2 s are exact,
+// so only one sqrt and two products round.  The retry loop only finds the
+// accepted words (the point's arithmetic, inlined at each test, ran up to
+// four times per wave).
+// N sites per lane: their chains of dependent multiplies and roots interleave,
+// and a retry call serves whichever site of a lane still needs one.
+template <int N>
+__device__ __forceinline__ void counter_draws(unsigned long long seed, uint32_t replica, uint32_t sweep,
+                                              const uint32_t (&site)[N], int constrain_to_x, double (&px)[N],
+                                              double (&py)[N], double (&pz)[N], double (&u)[N])
 {
     const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
-    uint32_t w[4] = {site, sweep, replica, 0u};
-    philox4x32_10(w, k0, k1);
-    u = ((double)(w[2] >> 5) * 67108864.0 + (double)(w[3] >> 6)) * (1.0 / 9007199254740992.0);
+    double x1[N], x2[N], S[N];
+    uint32_t w0[N];
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        uint32_t w[4] = {site[n], sweep, replica, 0u};
+        philox4x32_10(w, k0, k1);
+        u[n] = ((double)(w[2] >> 5) * 67108864.0 + (double)(w[3] >> 6)) * (1.0 / 9007199254740992.0);
+        x1[n] = disc_coordinate(w[0]);
+        x2[n] = disc_coordinate(w[1]);
+        S[n] = disc_norm2(x1[n], x2[n]);
+        w0[n] = w[0];
+    }
     if (constrain_to_x) {
-        uint32_t i = w[0] % 6u;
-        px = (i == 0) ? 1.0 : (i == 1) ? -1.0 : 0.0;
-        py = (i == 2) ? 1.0 : (i == 3) ? -1.0 : 0.0;
-        pz = (i == 4) ? 1.0 : (i == 5) ? -1.0 : 0.0;
+#pragma unroll
+        for (int n = 0; n < N; n++) {
+            const uint32_t i = w0[n] % 6u;
+            px[n] = (i == 0) ? 1.0 : (i == 1) ? -1.0 : 0.0;
+            py[n] = (i == 2) ? 1.0 : (i == 3) ? -1.0 : 0.0;
+            pz[n] = (i == 4) ? 1.0 : (i == 5) ? -1.0 : 0.0;
+        }
         return;
     }
-    // the point of candidate words (a0, a1) if it lies in the disc
-    auto disc = [&](uint32_t a0, uint32_t a1) -> bool {
-        const long long a = 2 * (long long)(a0 >> 6) + 1 - (1ll << 26);
-        const long long b = 2 * (long long)(a1 >> 6) + 1 - (1ll << 26);
-        const long long s = a * a + b * b;
-        if (s >= (1ll << 52)) return false;
-        const double x1 = (double)a * (1.0 / 67108864.0);
-        const double x2 = (double)b * (1.0 / 67108864.0);
-        const double S = (double)s * (1.0 / 4503599627370496.0);
-        const double r = __builtin_sqrt(1.0 - S);
-        px = (2.0 * x1) * r;
-        py = (2.0 * x2) * r;
-        pz = 1.0 - 2.0 * S;
-        return true;
-    };
-    if (disc(w[0], w[1])) return;
-    for (uint32_t k = 1; k <= 32; k++) {
-        uint32_t c[4] = {site, sweep, replica, k};
+    // (a lane's sites retry in order: site 0 until it has its point, then 1)
+    uint32_t k = 1;
+    for (;;) {
+        const bool two = N > 1 && S[0] < 1.0;   // site 0 is done
+        const double s = two ? S[N - 1] : S[0];
+        if (!(s >= 1.0)) break;
+        uint32_t c[4] = {two ? site[N - 1] : site[0], sweep, replica, k};
         philox4x32_10(c, k0, k1);
-        if (disc(c[0], c[1]) || disc(c[2], c[3])) return;
+        double y1 = disc_coordinate(c[0]), y2 = disc_coordinate(c[1]), T = disc_norm2(y1, y2);
+        const double v1 = disc_coordinate(c[2]), v2 = disc_coordinate(c[3]), V = disc_norm2(v1, v2);
+        if (T >= 1.0) { y1 = v1; y2 = v2; T = V; }
+        if (T >= 1.0 && k == 32) { y1 = 0.0; y2 = 0.0; T = 0.0; }   // 65 rejections in a row (p ~ 1e-43): (0, 0, 1)
+        k = T >= 1.0 ? k + 1 : 1;
+        if (two) { x1[N - 1] = y1; x2[N - 1] = y2; S[N - 1] = T; }
+        else { x1[0] = y1; x2[0] = y2; S[0] = T; }
     }
-    px = 0.0; py = 0.0; pz = 1.0;   // 65 rejections in a row: p ~ 1e-43
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        const double r = sqrt_unit(1.0 - S[n]);
+        px[n] = (2.0 * x1[n]) * r;
+        py[n] = (2.0 * x2[n]) * r;
+        pz[n] = 1.0 - 2.0 * S[n];
+    }
+}
+
+__device__ __forceinline__ void counter_draw(unsigned long long seed, uint32_t replica, uint32_t sweep, uint32_t site,
+                                             int constrain_to_x, double &px, double &py, double &pz, double &u)
+{
+    const uint32_t sites[1] = {site};
+    double x[1], y[1], z[1], v[1];
+    counter_draws<1>(seed, replica, sweep, sites, constrain_to_x, x, y, z, v);
+    px = x[0]; py = y[0]; pz = z[0]; u = v[0];
 }
 
 // Metropolis threshold: exp(-beta dE) > u  <=>  dE < -ln(u)/beta, and the
 // dE < 0 branch of src/starrynight-montecarlo-core.c:179 is covered because
 // the threshold is >= 0.  beta = +inf (T = 0) gives 0: only dE < 0 accepted.
-__device__ __forceinline__ double metropolis_threshold(double u, double beta)
+// rbeta = 1 / beta, rounded: the quotient is its product corrected by its own
+// residual, which is the correctly rounded quotient (Markstein 1990) while
+// nothing over- or underflows; a beta that could is divided by.
+__device__ __forceinline__ double metropolis_threshold(double u, double beta, double rbeta)
 {
     if (u <= 0.0 || beta <= 0.0) return __builtin_inf();
     if (__builtin_isinf(beta)) return 0.0;
-    return -log(u) / beta;
+    const double l = -log_unit(u);
+    if (!(beta > 1e-200 && beta < 1e200)) return l / beta;
+    const double q = l * rbeta;
+    return fma(fma(-q, beta, l), rbeta, q);
 }
 
 __device__ __forceinline__ int wrap_once(int v, int L)

@@ -181,6 +181,7 @@ __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_
 
     // proposal and Metropolis threshold of the chunk's site k (region index ri)
     const unsigned sweep = a.sweep_ctr[tile.replica];
+    const double rbeta = 1.0 / rep.beta;
     const long long tile_base = ((long long)tile.x0 * rep.Y + tile.y0) * rep.Z + tile.z0;
     auto draw = [&](int k, int ri) __attribute__((always_inline)) {
         const int iz = ri % RZs, q = ri / RZs;
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_
         prop[k] = px;
         prop[PS + k] = py;
         prop[2 * PS + k] = pz;
-        prop[3 * PS + k] = metropolis_threshold(u, rep.beta);
+        prop[3 * PS + k] = metropolis_threshold(u, rep.beta, rbeta);
     };
     // the first chunk's proposals are drawn while the staging loads are in
     // flight (its site list is read from global memory: the LDS copy is not

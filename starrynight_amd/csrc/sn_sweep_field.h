@@ -319,6 +319,7 @@ __global__ __launch_bounds__(kBlock) void field_sweep_kernel(FieldArgs fa, int f
     // while the staging loads are in flight and kept in registers until the
     // tile-order arrays exist ----
     const unsigned sweep = a.sweep_ctr[tile.replica];
+    const double rbeta = 1.0 / rep.beta;
     const long long tile_base = ((long long)tile.x0 * rep.Y + tile.y0) * rep.Z + tile.z0;
     const int ntile = sh.tx * sh.ty * sh.tz;
     constexpr int NPROP = (TWO_D ? kFieldMaxTile2D : kFieldMaxTile3D) / kBlock;
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(kBlock) void field_sweep_kernel(FieldArgs fa, int f
             const unsigned gsite = (unsigned)(tile_base + ((long long)lx * rep.Y + ly) * rep.Z + lz);
             double u;
             counter_draw(rep.seed, (uint32_t)tile.replica, sweep, gsite, rep.constrain_to_x, P.x, P.y, P.z, u);
-            P.thr = metropolis_threshold(u, rep.beta);
+            P.thr = metropolis_threshold(u, rep.beta, rbeta);
             P.kp = (lx * TYP + ly) * TZP + lz;
         }
     };

@@ -82,6 +82,7 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
     }
     // nearest-neighbour pairs come first in the table, so they sit in slot 0
     const double nnf = (part < t.npairs && t.pairs[part].nn) ? 1.0 : 0.0;
+    const double rbeta = 1.0 / rep.beta;
     const double J = rep.J, K = rep.K, E0 = rep.E[0], E1 = rep.E[1], E2 = rep.E[2];
     // uniform lengths: the cage-strain sum rides on the nearest-neighbour weight
     const double wn0 = (!MIXED && nnf != 0.0 && rep.L0 != 0.0) ? w[0] - J / (rep.L0 * rep.L0) : w[0];
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
                 prop[i] = px;
                 prop[PS + i] = py;
                 prop[2 * PS + i] = pz;
-                prop[3 * PS + i] = metropolis_threshold(u, rep.beta);
+                prop[3 * PS + i] = metropolis_threshold(u, rep.beta, rbeta);
             }
             __syncthreads();
             // ---- the run's colours, NG sites at a time (a colour's sites are
