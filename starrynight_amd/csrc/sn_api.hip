@@ -57,9 +57,8 @@ struct sn_ctx {
     RepDev *d_reps = nullptr;
     TileDev *d_tiles = nullptr;
     ShapeDev *d_shapes = nullptr;
-    int *d_class_start = nullptr, *d_class_ri = nullptr, *d_chunk_col = nullptr;
-    int *d_gsteps = nullptr, *d_gchunk = nullptr;   // gather kernel's step tables
-    int max_gsteps = 0;
+    int *d_sites = nullptr, *d_gsteps = nullptr;   // gather kernel's site and step tables
+    int max_gsteps = 0, max_chunks = 0;
     int *d_field_steps = nullptr, *d_tile_coord = nullptr;
     int max_steps = 0;   // longest step table of a tile shape (field kernel)
     int max_tile_padded = 0;   // largest padded tile (field kernel's tile-order arrays)
@@ -82,7 +81,6 @@ struct sn_ctx {
     void *d_stage = nullptr;
     size_t stage_cap = 0;
     double *d_scratch = nullptr;   // this device's `scratch` array (not owned)
-    int max_tile_sites = 0, max_cls = 0, max_chunks = 0;
     int gather_region = 0;   // largest staged region of the gather kernel (z rows padded, gather_zstride)
     int field_region = 0;   // largest staged region of the field kernel (z rows padded to odd)
     int *d_tile_list = nullptr;          // tile indices grouped by replica (tiled energy kernel)
@@ -269,9 +267,8 @@ static bool plan(const std::vector<ReplicaGeom> &geom, int rc, const sn_tuning &
 // dynamic LDS bytes of the per-phase gather kernel
 static size_t sweep_lds(const sn_ctx *c, bool mixed)
 {
-    size_t dbl = (size_t)((mixed ? 4 : 3) * c->gather_region + 4 * c->prop_chunk) * sizeof(double);
-    size_t ints = (size_t)(c->max_tile_sites + c->max_cls + 1 + 2 * (c->max_chunks + 1) +
-                           (c->max_gsteps + 1) * (c->blk / c->G + 1)) * sizeof(int);
+    size_t dbl = (size_t)((((mixed ? 4 : 3) * c->gather_region + 1) & ~1) + 4 * c->prop_chunk) * sizeof(double);
+    size_t ints = (size_t)((c->max_gsteps + 1) * (c->blk / c->G) + 2 * (c->max_chunks + 1)) * sizeof(int);
     return dbl + ints;
 }
 
@@ -572,6 +569,7 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     for (const Offset &o : pairs) hp.push_back(to_dev(o));
     for (const Offset &o : offs) ho.push_back(to_dev(o));
     c->npairs = (int)hp.size();
+    hp.resize(std::max<size_t>(hp.size(), kPairSlots), PairDev{});
     c->noff = (int)ho.size();
 
     // lanes per site and pairs per lane
@@ -678,29 +676,24 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     for (int r = 0; r < c->R; r++) rd.push_back(make_repdev(c->params[r], c->reps[r]));
     int st;
     if ((st = upload(c, &c->d_reps, rd))) return st;
-    std::vector<TileDev> td;
-    for (const Tile &t : c->sched.tiles) td.push_back({t.replica, t.x0, t.y0, t.z0, t.shape, 0, 0, 0});
-    if ((st = upload(c, &c->d_tiles, td))) return st;
     std::vector<ShapeDev> sd;
-    std::vector<int> cstart, cri, chunks, fsteps, tcoord, gsteps, gchunk;
+    std::vector<int> cri, cxyz, fsteps, tcoord, gsteps, sites_off, gstep_off, gsteps_n;
     const int NGg = blk / G;   // lane groups of the gather kernel
     constexpr int NG = kBlock / kFieldG;   // lane groups of the field kernel
     const int hz = c->two_d ? 0 : c->rc;
     for (const TileShape &s : c->sched.shapes) {
         ShapeDev d{};
         d.tx = s.tx; d.ty = s.ty; d.tz = s.tz; d.ncol = s.ncol;
-        d.nchunks = (int)s.chunk_start.size() - 1;
-        d.class_off = (int)cstart.size();
-        d.chunk_off = (int)chunks.size();
-        d.sites_off = (int)cri.size();
-        cstart.insert(cstart.end(), s.class_start.begin(), s.class_start.end());
-        // by fine colour: region index (tile + halo) and tile-local index of
-        // each site; by tile index: packed local coordinates
+        const int nchunks = (int)s.chunk_start.size() - 1;
+        sites_off.push_back((int)cri.size());
+        // by fine colour: region index (tile + halo) and packed local
+        // coordinates of each site; by tile index: packed local coordinates
         const int RY = s.ty + 2 * c->rc, RZ = s.tz + 2 * hz, RZs = gather_zstride(RZ);
         for (size_t k = 0; k < s.class_sites.size(); k++) {
             int li = s.class_sites[k];
             int lz = li % s.tz, ly = (li / s.tz) % s.ty, lx = li / (s.tz * s.ty);
             cri.push_back(((lx + c->rc) * RY + (ly + c->rc)) * RZs + (lz + hz));
+            cxyz.push_back(lx | (ly << 10) | (lz << 20));
         }
         c->gather_region = std::max(c->gather_region, (s.tx + 2 * c->rc) * RY * RZs);
         // field kernel: tile-order arrays use padded strides (z in 3D, y in
@@ -732,45 +725,57 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
             }
         }
         c->max_steps = std::max(c->max_steps, d.nsteps);
-        chunks.insert(chunks.end(), s.chunk_start.begin(), s.chunk_start.end());
-        // gather kernel steps: per proposal chunk, each colour in blocks of NGg
-        // sites; per step a barrier flag (last block of the colour) and NGg
-        // entries (region index | slot in the chunk's proposals << 16, or -1)
-        d.gstep_off = (int)gsteps.size();
-        d.gchunk_off = (int)gchunk.size();
+        // gather kernel steps: per proposal chunk (its first step and site in
+        // gchunk), each colour in blocks of NGg sites, an entry (step_entry) per
+        // lane group; one idle row at the end
+        gstep_off.push_back((int)gsteps.size());
+        std::vector<int> gchunk;
+        const int *ri = cri.data() + sites_off.back();
         int nst = 0;
-        for (int ch = 0; ch < d.nchunks; ch++) {
-            gchunk.push_back(nst);
+        for (int ch = 0; ch < nchunks; ch++) {
             const int c0 = s.chunk_start[ch], c1 = s.chunk_start[ch + 1];
             const int s0 = s.class_start[c0];
+            gchunk.push_back(nst);
+            gchunk.push_back(s0);
             for (int col = c0; col < c1; col++) {
                 const int a0 = s.class_start[col], a1 = s.class_start[col + 1];
                 for (int b0 = a0; b0 < a1; b0 += NGg) {
-                    gsteps.push_back(b0 + NGg >= a1 ? 1 : 0);
+                    const bool last = b0 + NGg >= a1;
                     for (int g = 0; g < NGg; g++)
-                        gsteps.push_back(b0 + g < a1 ? (cri[d.sites_off + b0 + g] | ((b0 + g - s0) << 16)) : -1);
+                        gsteps.push_back(b0 + g < a1 ? step_entry(ri[b0 + g], b0 + g - s0, last, false)
+                                                     : step_entry(ri[0], 0, last, true));
                     nst++;
                 }
             }
         }
         gchunk.push_back(nst);
-        d.gsteps_n = nst;
+        gchunk.push_back(s.class_start[s.ncol]);
+        for (int g = 0; g < NGg; g++) gsteps.push_back(step_entry(ri[0], 0, false, true));
+        gsteps.insert(gsteps.end(), gchunk.begin(), gchunk.end());
+        c->max_chunks = std::max(c->max_chunks, nchunks);
+        gsteps_n.push_back(nst);
         c->max_gsteps = std::max(c->max_gsteps, nst);
-        c->max_tile_sites = std::max(c->max_tile_sites, s.tx * s.ty * s.tz);
         const int RZp = c->two_d ? RZ : (RZ | 1);
         c->field_region = std::max(c->field_region, (s.tx + 2 * c->rc) * RY * RZp);
-        c->max_cls = std::max(c->max_cls, s.ncol);
-        c->max_chunks = std::max(c->max_chunks, d.nchunks);
         sd.push_back(d);
     }
     if ((st = upload(c, &c->d_shapes, sd))) return st;
-    if ((st = upload(c, &c->d_class_start, cstart))) return st;
-    if ((st = upload(c, &c->d_class_ri, cri))) return st;
+    std::vector<TileDev> td;
+    for (const Tile &t : c->sched.tiles) {
+        const TileShape &s = c->sched.shapes[t.shape];
+        const RepHost &h = c->reps[t.replica];
+        TileDev d{t.replica, t.x0, t.y0, t.z0, t.shape, h.X, h.Y, h.Z, h.base,
+                  s.tx | (s.ty << 10) | (s.tz << 20), sites_off[t.shape], 0, gstep_off[t.shape], gsteps_n[t.shape], (int)s.chunk_start.size() - 1};
+        const int nch = d.nchunks;
+        auto first = [&](int ch) { return s.class_start[s.chunk_start[std::min(ch, nch)]]; };
+        d.first_chunks = (first(1) - first(0)) | ((first(2) - first(1)) << 16);
+        td.push_back(d);
+    }
+    if ((st = upload(c, &c->d_tiles, td))) return st;
+    if ((st = upload(c, &c->d_sites, cxyz))) return st;
     if ((st = upload(c, &c->d_field_steps, fsteps))) return st;
     if ((st = upload(c, &c->d_tile_coord, tcoord))) return st;
-    if ((st = upload(c, &c->d_chunk_col, chunks))) return st;
     if ((st = upload(c, &c->d_gsteps, gsteps))) return st;
-    if ((st = upload(c, &c->d_gchunk, gchunk))) return st;
     if ((st = upload(c, &c->d_pairs, hp))) return st;
     if ((st = upload(c, &c->d_offs, ho))) return st;
     std::vector<unsigned> zeros_u(c->R, 0u);
@@ -839,8 +844,8 @@ int sn_destroy(sn_ctx *c)
     if (!c) return SN_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     free_graph(c);
-    void *bufs[] = {c->d_lat, c->d_reps, c->d_tiles, c->d_shapes, c->d_class_start, c->d_class_ri,
-                    c->d_field_steps, c->d_tile_coord, c->d_chunk_col, c->d_gsteps, c->d_gchunk, c->d_pairs,
+    void *bufs[] = {c->d_lat, c->d_reps, c->d_tiles, c->d_shapes, c->d_sites,
+                    c->d_field_steps, c->d_tile_coord, c->d_gsteps, c->d_pairs,
                     c->d_offs, c->d_sweep,
                     c->d_counters, c->d_partials, c->d_result, c->d_radial, c->d_radial_bins,
                     c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_sites,
@@ -1035,15 +1040,11 @@ static SweepArgs sweep_args(sn_ctx *c)
 {
     SweepArgs a;
     a.lat = c->d_lat; a.reps = c->d_reps; a.tiles = c->d_tiles; a.shapes = c->d_shapes;
-    a.class_start = c->d_class_start; a.class_ri = c->d_class_ri; a.chunk_col = c->d_chunk_col;
-    a.gsteps = c->d_gsteps; a.gchunk = c->d_gchunk;
-    a.max_gsteps = c->max_gsteps; a.max_chunks = c->max_chunks;
+    a.sites = c->d_sites; a.gsteps = c->d_gsteps;
     a.prop_stride = c->prop_chunk;
     a.pairs = c->d_pairs; a.sweep_ctr = c->d_sweep; a.counters = c->d_counters;
     a.npairs = c->npairs; a.rc = c->rc; a.two_d = c->two_d ? 1 : 0;
     a.max_region = c->gather_region;
-    a.max_tile_sites = c->max_tile_sites;
-    a.max_cls = c->max_cls;
     return a;
 }
 

@@ -16,16 +16,21 @@ struct RepDev {
     int constrain_to_x, pad;
 };
 
+// One tile of the schedule, with its replica's size and its own: the staging
+// loads of a tile depend on this record alone, not on a chain of tables.
 struct TileDev {
-    int replica, x0, y0, z0, shape, pad0, pad1, pad2;
+    int replica, x0, y0, z0, shape, X, Y, Z;
+    long long base;        // first site of the replica in the lattice buffer
+    int size;              // tx | ty << 10 | tz << 20
+    int sites_off, first_chunks;   // the shape's site list; sites of its first two proposal chunks, n0 | n1 << 16
+    int gstep_off, gsteps_n, nchunks;   // the shape's step table, its steps and proposal chunks
 };
+static_assert(sizeof(TileDev) == 64, "one scalar load");
 
 struct ShapeDev {
     int tx, ty, tz, ncol;
-    int nchunks, class_off, chunk_off, sites_off;
     int nsteps, step_off;     // field kernel's step table (see sn_sweep_field.h)
     int typ, tzp, coord_off;  // field kernel's padded tile-order strides and coordinate table
-    int gstep_off, gchunk_off, gsteps_n;   // gather kernel's step table (see sn_kernels.h)
 };
 
 // z stride of the gather kernel's staged region.  A row of a multiple of 8

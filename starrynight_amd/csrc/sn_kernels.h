@@ -12,26 +12,32 @@
 namespace sn {
 
 constexpr int kBlock = 256;   // threads per workgroup of the tile sweep
+constexpr int kPairSlots = 512;   // largest lanes x pairs per lane of a gather instance
 
 struct SweepArgs {
     double4 *lat;
     const RepDev *reps;
     const TileDev *tiles;
     const ShapeDev *shapes;
-    const int *class_start;   // per shape: ncol + 1 entries (offsets into class_ri)
-    const int *class_ri;      // per shape: LDS region index of each tile site, by fine colour
-    const int *chunk_col;     // per shape: nchunks + 1 colour indices
     const PairDev *pairs;
     const unsigned *sweep_ctr;
     unsigned long long *counters;  // 2 per tile: accepted, rejected (accumulated over sweeps)
-    const int *gsteps;        // per shape (gstep_off): per step, barrier flag + BLK / G entries
-                              // (region index | proposal slot << 16, or -1)
-    const int *gchunk;        // per shape (gchunk_off): first step of each proposal chunk (nchunks + 1)
-    int npairs, rc, two_d, max_region;
-    int max_tile_sites, max_cls;   // sizes of the LDS copies of the shape tables
-    int max_gsteps, max_chunks;
+    const int *sites;         // per shape (TileDev.sites_off): tile sites by fine colour, packed lx | ly << 10 | lz << 20
+    const int *gsteps;        // per shape (TileDev.gstep_off): per step BLK / G entries (step_entry), an idle row, then
+                              // the first step and the first site of each proposal chunk (nchunks + 1 of both)
+    int npairs;               // (the table is padded with zero pairs to kPairSlots)
+    int rc, two_d, max_region;
     int prop_stride;          // proposal slots per chunk (<= kBlock)
 };
+
+// Entry of a lane group in the step table: the site's region index, its slot
+// in the chunk's proposals, a flag on a colour's last step (it ends with the
+// barrier), and the sign bit for a group without a site.
+constexpr int kStepBarrier = 1 << 30, kStepIdle = (int)0x80000000u;
+__host__ __device__ inline int step_entry(int ri, int slot, bool last, bool idle)
+{
+    return ri | (slot << 16) | (last ? kStepBarrier : 0) | (idle ? kStepIdle : 0);
+}
 
 // DPP lane exchange of a double (two 32-bit moves); CTRL is a dpp_ctrl code.
 template <int CTRL>
@@ -43,6 +49,15 @@ __device__ __forceinline__ double dpp_f64(double v)
     lo = __builtin_amdgcn_mov_dpp(lo, CTRL, 0xF, 0xF, true);
     hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, true);
     return __hiloint2double(hi, lo);
+}
+
+// Lane C of the aligned quad (G < 16) or of the row of 16 lanes (G >= 16, one
+// instruction) in every lane of it.
+template <int C, int G>
+__device__ __forceinline__ double lane_bcast(double v)
+{
+    if constexpr (G >= 16) return __builtin_amdgcn_update_dpp(v, v, 0x150 + C, 0xF, 0xF, true);
+    else return dpp_f64<C * 0x55>(v);
 }
 
 // v + v[lane ^ 16] (ROWS = 16) or v + v[lane ^ 32] (ROWS = 32) in every lane,
@@ -82,11 +97,14 @@ __device__ __forceinline__ double group_sum_dpp(double v)
     return v;
 }
 
+// -3 w n of a lane's pairs (present only where the kernel keeps it)
+template <int N, bool ON> struct PairTerm { double x[N], y[N], z[N]; };
+template <int N> struct PairTerm<N, false> {};
+
 // One workgroup updates one tile: stage tile + halo in LDS, draw the
 // proposals of all tile sites, run the fine colours one after another (G lanes
 // share one site's neighbour sum, NPL +-r pairs per lane), write the tile back.
-__device__ __forceinline__ int s_gchunk_total(const ShapeDev &sh) { return sh.gsteps_n; }
-
+//
 // BLK threads per workgroup (256 or 512); proposals are drawn in chunks of at
 // most prop_stride (<= kBlock) sites.  The staged x, y, z arrays are read by
 // separate instructions: a read2 of x and y at a stride that is a multiple of
@@ -95,27 +113,21 @@ __device__ __forceinline__ int s_gchunk_total(const ShapeDev &sh) { return sh.gs
 // MRC > 0 fixes the stride of the staged arrays at compile time (the launch's
 // max_region must equal it, and its prop_stride kBlock): the y and z reads then
 // take immediate LDS offsets from the x address instead of an address add each
-// (measured 2% at 8^3 tiles), and so do the proposal reads.
-// -3 w n of a lane's pairs (present only where the kernel keeps it)
-template <int N, bool ON> struct PairTerm { double x[N], y[N], z[N]; };
-template <int N> struct PairTerm<N, false> {};
-
+// (measured 2% at 8^3 tiles).
 template <int G, int NPL, bool MIXED, int BLK, int MRC = 0>
 __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_tile, int ntiles)
 {
-    extern __shared__ double smem[];
+    static_assert(G * NPL <= kPairSlots, "the pair table covers every lane's slots");
+    extern __shared__ __align__(16) double smem[];
     const int tid = threadIdx.x;
     const int b = blockIdx.x;
     // Consecutive tiles (spatial neighbours sharing halo sites) go to the same
     // XCD: the hardware deals workgroups to the 8 XCDs round-robin.
     const int t = (ntiles % 8 == 0) ? (b % 8) * (ntiles / 8) + b / 8 : b;
     const TileDev tile = a.tiles[first_tile + t];
-    const RepDev rep = a.reps[tile.replica];
-    const ShapeDev sh = a.shapes[tile.shape];
     const int hx = a.rc, hy = a.rc, hz = a.two_d ? 0 : a.rc;
-    const int RY = sh.ty + 2 * hy, RZ = sh.tz + 2 * hz;
-    const int RX = sh.tx + 2 * hx;
-    const int region = RX * RY * RZ;                       // sites staged
+    const int tx = tile.size & 1023, ty = (tile.size >> 10) & 1023, tz = tile.size >> 20;
+    const int RX = tx + 2 * hx, RY = ty + 2 * hy, RZ = tz + 2 * hz;
     const int RZs = gather_zstride(RZ);                    // z stride in LDS (>= RZ)
 
     const int MR = MRC > 0 ? MRC : a.max_region;          // stride of the staged arrays
@@ -130,131 +142,179 @@ __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_
     double *sy = MIXED ? sx + 1 : sx + MR;                 // y of site i at sy[ZS * i]
     double *sz = sx + 2 * MR;                              // z of site i at sz[ZS * i]
     double *sl = sz + 1;                                   // L of site i at sl[2 * i] (MIXED only)
-    double *prop = sz + ZS * MR;                           // 4 x prop_stride: px, py, pz, threshold
+    // proposals: px, py, pz and threshold of slot k at prop[4 k]
+    double *prop = sx + (((MIXED ? 4 : 3) * MR + 1) & ~1);
     const int PS = MRC > 0 ? kBlock : a.prop_stride;        // (fixed-stride launches draw chunks of kBlock)
-    int *s_ri = (int *)(prop + 4 * PS);                    // region index of class sites
-    int *s_cls = s_ri + a.max_tile_sites;                  // class starts, then chunk colours
-    int *s_chunk = s_cls + a.max_cls + 1;
-    int *s_gchunk = s_chunk + a.max_chunks + 1;            // first step of each chunk
-    int *s_gstep = s_gchunk + a.max_chunks + 1;            // step table
-    constexpr int SW = BLK / G + 1;                        // ints per step
+    int *s_gstep = (int *)(prop + 4 * PS);                 // step table and chunk table
+    constexpr int SW = BLK / G;                            // entries per step
 
-    // ---- shape tables into LDS ----
-    const int ntile = sh.tx * sh.ty * sh.tz;
-    for (int i = tid; i < ntile; i += BLK) s_ri[i] = a.class_ri[sh.sites_off + i];
-    for (int i = tid; i <= sh.ncol; i += BLK) s_cls[i] = a.class_start[sh.class_off + i];
-    for (int i = tid; i <= sh.nchunks; i += BLK) {
-        s_chunk[i] = a.chunk_col[sh.chunk_off + i];
-        s_gchunk[i] = a.gchunk[sh.gchunk_off + i];
-    }
-    for (int i = tid; i < s_gchunk_total(sh) * SW; i += BLK) s_gstep[i] = a.gsteps[sh.gstep_off + i];
+    const RepDev rep = a.reps[tile.replica];
+    const unsigned sweep = a.sweep_ctr[tile.replica];
+    const long long tile_base = ((long long)tile.x0 * tile.Y + tile.y0) * tile.Z + tile.z0;
 
-    // ---- this lane's share of the neighbour pairs, held in registers (loaded
-    // first: their latency overlaps the staging) ----
+    const double rbeta = 1.0 / rep.beta;
+    auto global_site = [&](int xyz) __attribute__((always_inline)) {   // of packed tile coordinates
+        const int lx = xyz & 1023, ly = (xyz >> 10) & 1023, lz = xyz >> 20;
+        return (uint32_t)(tile_base + ((long long)lx * tile.Y + ly) * tile.Z + lz);
+    };
+    // This lane's proposal slot in chunk ch (512 threads: alternate halves of
+    // the workgroup, so the first two chunks are drawn side by side)
+    auto slot_of = [&](int ch) __attribute__((always_inline)) { return tid - (BLK > kBlock ? (ch & 1) * kBlock : 0); };
+    const int k0 = slot_of(0), k1 = slot_of(1);
+    const int n0 = tile.first_chunks & 0xFFFF, n1 = tile.first_chunks >> 16;
+    const bool draw0 = k0 < n0, draw1 = k1 >= 0 && k1 < n1;   // (k0 is never negative)
+    int xyz0 = draw0 ? a.sites[tile.sites_off + k0] : 0;
+    int xyz1 = draw1 ? a.sites[tile.sites_off + n0 + k1] : 0;
+    // the step table's first entries, on their way to LDS
+    constexpr int NT = 4;
+    const int nstep = (tile.gsteps_n + 1) * SW + 2 * (tile.nchunks + 1);
+    int tab[NT];
+#pragma unroll
+    for (int k = 0; k < NT; k++) tab[k] = tid + k * BLK < nstep ? a.gsteps[tile.gstep_off + tid + k * BLK] : 0;
+
+    // ---- this lane's share of the neighbour pairs, held in registers ----
     const int part = tid % G;
     const int group = tid / G;
     int dl[NPL];
-    double nx[NPL], ny[NPL], nz[NPL], w[NPL], w3[NPL];
+    double nx[NPL], ny[NPL], nz[NPL], w[NPL], w3[NPL], nnf = 0.0;
 #pragma unroll
     for (int m = 0; m < NPL; m++) {
-        int j = part + m * G;
-        if (j < a.npairs) {
-            PairDev p = a.pairs[j];
-            dl[m] = (p.dx * RY + p.dy) * RZs + p.dz;
-            nx[m] = p.nx; ny[m] = p.ny; nz[m] = p.nz; w[m] = p.w; w3[m] = -3.0 * p.w;
-        } else {
-            dl[m] = 0; nx[m] = 0.0; ny[m] = 0.0; nz[m] = 0.0; w[m] = 0.0; w3[m] = 0.0;
+        const PairDev p = a.pairs[part + m * G];   // (padded with zero pairs to every G x NPL)
+        dl[m] = (p.dx * RY + p.dy) * RZs + p.dz;
+        nx[m] = p.nx; ny[m] = p.ny; nz[m] = p.nz; w[m] = p.w; w3[m] = -3.0 * p.w;
+        // nearest-neighbour pairs come first in the table, so they sit in slot 0
+        if (m == 0) nnf = p.nn ? 1.0 : 0.0;
+    }
+    // ---- load tile + halo (periodic wrap).  A lane keeps its (y, z) and walks
+    // the x planes, so a load's address costs an add (stepping every lane
+    // through the region's mixed radix cost 65 instructions a load).  A launch
+    // finds the L2 empty and these loads take microseconds: NV of them per lane
+    // (all of a fixed-stride tile's 14 planes) are issued before anything
+    // waits, behind the few loads that the draws below need (loads return in
+    // order), and unconditionally (past the last plane: the last one again), so
+    // that the wait for the earlier loads can count them ----
+    constexpr int NV = MRC > 0 ? 14 : 8;
+    const double4 *lat = a.lat + tile.base;
+    const int rows = RY * RZ;
+    const int per = rows < BLK ? BLK / rows : 1;   // planes loaded by one pass of the workgroup
+    double4 v[NV];
+    struct Row {
+        int px, lds;        // first plane; region index of plane 0
+        const double4 *src; // plane 0 of the lattice
+        bool on;
+    };
+    // the lane's row in sub-pass s (planes of more than BLK rows take several)
+    auto row_of = [&](int s) __attribute__((always_inline)) {
+        Row r;
+        const int q = tid + s * BLK;
+        r.px = q / rows;
+        const int k = min(q - r.px * rows, rows - 1), iy = k / RZ, iz = k - iy * RZ;
+        r.on = per > 1 ? r.px < per : q < rows;
+        if (per == 1) r.px = 0;
+        r.lds = iy * RZs + iz;
+        r.src = lat + (long long)wrap_once(tile.y0 - hy + iy, tile.Y) * tile.Z + wrap_once(tile.z0 - hz + iz, tile.Z);
+        return r;
+    };
+    auto load_planes = [&](const Row &r, int x) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const int ix = min(x + k * per + r.px, RX - 1);
+            v[k] = r.src[(long long)(wrap_once(tile.x0 - hx + ix, tile.X) * (tile.Y * tile.Z))];
+        }
+    };
+    Row row = row_of(0);
+    load_planes(row, 0);
+
+    // The first two chunks' proposals are drawn while the tile's loads are in
+    // flight (the fence keeps the loads above them); the second chunk's wait in
+    // registers for their slots.
+    double2 nxy, nzt;
+    asm volatile("" : "+v"(xyz0), "+v"(xyz1) : : "memory");
+#pragma unroll
+    for (int k = 0; k < NT; k++)
+        if (tid + k * BLK < nstep) s_gstep[tid + k * BLK] = tab[k];
+    {
+        // 256 threads: both sites of a lane together; 512: one each
+        constexpr int ND = BLK > kBlock ? 1 : 2;
+        uint32_t site[ND];
+        double px[ND], py[ND], pz[ND], u[ND];
+        site[0] = global_site(ND == 1 && draw1 ? xyz1 : xyz0);
+        site[ND - 1] = ND == 1 ? site[0] : global_site(xyz1);
+        if (draw0 || draw1) counter_draws<ND>(rep.seed, (uint32_t)tile.replica, sweep, site, rep.constrain_to_x, px, py, pz, u);
+        if (draw0) {
+            ((double2 *)prop)[2 * k0] = make_double2(px[0], py[0]);
+            ((double2 *)prop)[2 * k0 + 1] = make_double2(pz[0], metropolis_threshold(u[0], rep.beta, rbeta));
+        }
+        if (draw1) {
+            nxy = make_double2(px[ND - 1], py[ND - 1]);
+            nzt = make_double2(pz[ND - 1], metropolis_threshold(u[ND - 1], rep.beta, rbeta));
         }
     }
+    for (int i = tid + NT * BLK; i < nstep; i += BLK) s_gstep[i] = a.gsteps[tile.gstep_off + i];
+
+    // ---- staged sites into LDS ----
+    for (int sub = 0;;) {
+        for (int x = 0;;) {
+#pragma unroll
+            for (int k = 0; k < NV; k++) {
+                const int ix = x + k * per + row.px;
+                if (row.on && ix < RX) {
+                    const int i = ix * (RY * RZs) + row.lds;
+                    if (MIXED) {
+                        ((double2 *)sx)[i] = make_double2(v[k].x, v[k].y);
+                        ((double2 *)sz)[i] = make_double2(v[k].z, v[k].w);
+                    } else {
+                        sx[i] = v[k].x; sy[i] = v[k].y; sz[i] = v[k].z;
+                    }
+                }
+            }
+            x += NV * per;
+            if (x >= RX) break;
+            load_planes(row, x);
+        }
+        if (++sub * BLK >= rows) break;
+        row = row_of(sub);
+        load_planes(row, 0);
+    }
+
     // TN: t = -3 w n per pair in registers, one multiply fewer per pair for
     // three more registers.  Only the fixed-stride instances take it: their
     // LDS (>= 66 KB) allows two workgroups per CU, so up to 256 VGPRs cost no
     // occupancy, while smaller tiles run three workgroups per CU (<= 168).
     constexpr bool TN = MRC > 0;
+    // the field term, and with it K's, ride on the group's first lane
+    const double J = rep.J, K = rep.K;
+    const double E0 = part == 0 ? rep.E[0] : 0.0, E1 = part == 0 ? rep.E[1] : 0.0, E2 = part == 0 ? rep.E[2] : 0.0;
+    // A site's own data, one component a lane: lane c of each quad reads p'_c
+    // and p_c (c < 3), lane 3 the threshold and (mixed lengths) the length, and
+    // hands its difference to the others by DPP: two LDS reads a step instead
+    // of the seven doubles every lane needs; an accepted site's components are
+    // written by three lanes at once.
+    const int comp = part & 3;
+    double *own = MIXED ? sx + (comp >> 1) * 2 * MR + (comp & 1) : sx + (comp < 3 ? comp : 2) * MR;
+    const double Kp = part < 2 ? K : 0.0;
+    // Uniform lengths: L0^2 and the cage strain ride on the weights, w' = L0^2 w
+    // (- J for nearest neighbours), so no separate g is accumulated.  Mixed
+    // lengths keep g (L_j sits inside h).
+    if constexpr (!MIXED) {
+        const double LL = rep.L0 * rep.L0;
+#pragma unroll
+        for (int m = 0; m < NPL; m++) { w[m] *= LL; w3[m] *= LL; }
+        w[0] -= nnf * J;
+    }
     PairTerm<NPL, TN> t3;
     if constexpr (TN) {
 #pragma unroll
         for (int m = 0; m < NPL; m++) { t3.x[m] = w3[m] * nx[m]; t3.y[m] = w3[m] * ny[m]; t3.z[m] = w3[m] * nz[m]; }
     }
-    // nearest-neighbour pairs come first in the table, so they sit in slot 0
-    const double nnf = (part < a.npairs && a.pairs[part].nn) ? 1.0 : 0.0;
-
-    // proposal and Metropolis threshold of the chunk's site k (region index ri)
-    const unsigned sweep = a.sweep_ctr[tile.replica];
-    const double rbeta = 1.0 / rep.beta;
-    const long long tile_base = ((long long)tile.x0 * rep.Y + tile.y0) * rep.Z + tile.z0;
-    auto draw = [&](int k, int ri) __attribute__((always_inline)) {
-        const int iz = ri % RZs, q = ri / RZs;
-        const int iy = q % RY, ix = q / RY;
-        const unsigned gsite = (unsigned)(tile_base + ((long long)(ix - hx) * rep.Y + (iy - hy)) * rep.Z + (iz - hz));
-        double px, py, pz, u;
-        counter_draw(rep.seed, (uint32_t)tile.replica, sweep, gsite, rep.constrain_to_x, px, py, pz, u);
-        prop[k] = px;
-        prop[PS + k] = py;
-        prop[2 * PS + k] = pz;
-        prop[3 * PS + k] = metropolis_threshold(u, rep.beta, rbeta);
-    };
-    // the first chunk's proposals are drawn while the staging loads are in
-    // flight (its site list is read from global memory: the LDS copy is not
-    // ready before the barrier)
-    const int n0 = a.class_start[sh.class_off + a.chunk_col[sh.chunk_off + 1]];
-    const int ri0 = tid < n0 ? a.class_ri[sh.sites_off + tid] : 0;
-    bool drawn = false;
-
-    // ---- stage tile + halo (periodic wrap), 4 loads in flight per lane ----
-    const double4 *lat = a.lat + rep.base;
-    {
-        // mixed-radix position of element tid, and the step of BLK elements
-        int iz = tid % RZ, q = tid / RZ, iy = q % RY, ix = q / RY;
-        const int sz_ = BLK % RZ, q2 = BLK / RZ, sy_ = q2 % RY, sx_ = q2 / RY;
-        for (int base = tid; base < region; base += 4 * BLK) {
-            double4 v[4];
-            int idx[4], pidx[4];
+    const bool writer = part < 3 && (MIXED || rep.L0 != 0.0);   // vacancies never move and are not counted
+    unsigned nacc = 0, nvis = 0;   // accepted (on a group's first lane), visited
+    __shared__ unsigned s_cnt[2];
+    if (tid < 2) s_cnt[tid] = 0;
+    // the pair registers are loaded by now: waiting for them here keeps the
+    // waits out of the step loop
 #pragma unroll
-            for (int k = 0; k < 4; k++) {
-                idx[k] = base + k * BLK;
-                pidx[k] = RZs == RZ ? idx[k] : (ix * RY + iy) * RZs + iz;
-                if (idx[k] < region) {
-                    int gx = wrap_once(tile.x0 - hx + ix, rep.X);
-                    int gy = wrap_once(tile.y0 - hy + iy, rep.Y);
-                    int gz = wrap_once(tile.z0 - hz + iz, rep.Z);
-                    v[k] = lat[((long long)gx * rep.Y + gy) * rep.Z + gz];
-                }
-                iz += sz_; iy += sy_; ix += sx_;
-                if (iz >= RZ) { iz -= RZ; iy++; }
-                if (iy >= RY) { iy -= RY; ix++; }
-            }
-            if (!drawn) {
-                // after this batch's loads have issued (the fence keeps them
-                // above it), before their data is needed
-                drawn = true;
-                int r0 = ri0;
-                asm volatile("" : "+v"(r0) : : "memory");
-                if (tid < n0) draw(tid, r0);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                if (idx[k] < region) {
-                    if (MIXED) {
-                        double2 xy, zl;
-                        xy.x = v[k].x; xy.y = v[k].y; zl.x = v[k].z; zl.y = v[k].w;
-                        ((double2 *)sx)[pidx[k]] = xy;
-                        ((double2 *)sz)[pidx[k]] = zl;
-                    } else {
-                        sx[pidx[k]] = v[k].x; sy[pidx[k]] = v[k].y; sz[pidx[k]] = v[k].z;
-                    }
-                }
-            }
-        }
-    }
-    if (!drawn && tid < n0) draw(tid, ri0);   // lanes past a small region's end
-
-    const double J = rep.J, K = rep.K, E0 = rep.E[0], E1 = rep.E[1], E2 = rep.E[2];
-    // Uniform lengths: the cage-strain sum rides on the nearest-neighbour
-    // pair's weight, h' = h - J / L0^2 g, so the partial is L0^2 dp.h' and no
-    // separate g is accumulated.  Mixed lengths keep g (L_j sits inside h).
-    const double wn0 = (!MIXED && nnf != 0.0 && rep.L0 != 0.0) ? w[0] - J / (rep.L0 * rep.L0) : w[0];
-    unsigned nacc = 0, nrej = 0;
+    for (int m = 0; m < NPL; m++) asm volatile("" : "+v"(dl[m]), "+v"(nx[m]), "+v"(ny[m]), "+v"(nz[m]), "+v"(w[m]));
     __syncthreads();
     if (MIXED) {
         // vacant sites (length 0) leave the tile's step table: the reference
@@ -265,57 +325,63 @@ __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_
         // vacant, 512 threads: 1.89e9 -> 2.29e9 (dropping) -> 2.43e9 (packing)
         // site-updates/s.  Packing a colour's sites across its steps instead
         // measured 2.36e9.
-        for (int i = tid; i < s_gchunk_total(sh) * SW; i += BLK) {
-            const int e_ = s_gstep[i];
-            if (i % SW != 0 && e_ >= 0 && sl[2 * (e_ & 0xFFFF)] == 0.0) s_gstep[i] = -1;
-        }
+        for (int i = tid; i < tile.gsteps_n * SW; i += BLK)
+            if (sl[2 * (s_gstep[i] & 0xFFFF)] == 0.0) s_gstep[i] |= kStepIdle;
         __syncthreads();
-        for (int st_ = tid; st_ < s_gchunk_total(sh); st_ += BLK) {
-            int *row = s_gstep + st_ * SW + 1;
+        for (int st_ = tid; st_ < tile.gsteps_n; st_ += BLK) {
+            int *row = s_gstep + st_ * SW;
+            const int idle = row[0] | kStepIdle;   // with the row's barrier flag
             int k = 0;
-            for (int g = 0; g < SW - 1; g++) {
+            for (int g = 0; g < SW; g++) {
                 const int e_ = row[g];
                 if (e_ >= 0) row[k++] = e_;
             }
-            for (; k < SW - 1; k++) row[k] = -1;
+            for (; k < SW; k++) row[k] = idle;
         }
         __syncthreads();
     }
 
-    for (int ch = 0; ch < sh.nchunks; ch++) {
-        const int c0 = s_chunk[ch], c1 = s_chunk[ch + 1];
-        const int s0 = s_cls[c0], s1 = s_cls[c1];
-        // ---- proposals of this chunk's sites: one site per lane (the first
-        // chunk's were drawn during staging) ----
-        if (ch > 0 && tid < s1 - s0) draw(tid, s_ri[s0 + tid]);
-        if (ch > 0) __syncthreads();
+    const int *chunk = s_gstep + (tile.gsteps_n + 1) * SW;
+    for (int ch = 0; ch < tile.nchunks; ch++) {
+        const int st0 = __builtin_amdgcn_readfirstlane(chunk[2 * ch]);
+        const int st1 = __builtin_amdgcn_readfirstlane(chunk[2 * ch + 2]);
+        if (ch > 0) {
+            // the proposals drawn ahead take the slots (the last step of a
+            // chunk ended with the barrier), then the following chunk's are drawn
+            const int s0 = chunk[2 * ch + 1], s1 = chunk[2 * ch + 3], k = slot_of(ch);
+            if (k >= 0 && k < s1 - s0) {
+                ((double2 *)prop)[2 * k] = nxy;
+                ((double2 *)prop)[2 * k + 1] = nzt;
+            }
+            if (ch + 1 < tile.nchunks) {
+                const int s2 = chunk[2 * ch + 5], kn = slot_of(ch + 1);
+                if (kn >= 0 && kn < s2 - s1) {
+                    double u;
+                    counter_draw(rep.seed, (uint32_t)tile.replica, sweep, global_site(a.sites[tile.sites_off + s1 + kn]),
+                                 rep.constrain_to_x, nxy.x, nxy.y, nzt.x, u);
+                    nzt.y = metropolis_threshold(u, rep.beta, rbeta);
+                }
+            }
+            __syncthreads();
+        }
         // this chunk's steps: every group decides one site per step; a step
         // holds sites of one colour and a colour's last step ends with the
-        // barrier.  The next step's entry and flag load with this step's data.
-        const int st0 = s_gchunk[ch], st1 = s_gchunk[ch + 1];
-        // (the LDS table has one spare row, so the read one past a chunk's last
-        // step stays in the allocation; its value is never used)
-        int e = s_gstep[st0 * SW + 1 + group];
-        int flag = s_gstep[st0 * SW];
+        // barrier.  The next step's entry loads with this step's data (the LDS
+        // table has one spare row, whose value is never used).
+        int e = s_gstep[st0 * SW + group];
         for (int st = st0; st < st1; st++) {
             // a group without a site this step (a short colour) skips the step:
             // its lanes issue no LDS reads (the group's lanes are whole DPP rows,
             // so the reduction of the active groups is unaffected)
-            const bool active = e >= 0;
-            const int ri = e & 0xFFFF;
-            const int pq = e >> 16;
-            const int e_next = s_gstep[(st + 1) * SW + 1 + group];
-            const int flag_next = s_gstep[(st + 1) * SW];
-            if (active) {
-                double hx_, hy_, hz_;
-                double gx_, gy_, gz_;
-                // every LDS read of the step is issued before the first use, so
-                // the step waits for LDS latency once, not once per pair
+            const int e_next = s_gstep[(st + 1) * SW + group];
+            if (e >= 0) {
+                const int ri = e & 0xFFFF, pq = (e >> 16) & 0xFF;
+                double hx_, hy_, hz_, gx_, gy_, gz_;
                 double ax[NPL], ay[NPL], az[NPL], bx[NPL], by[NPL], bz[NPL], la[NPL], lb[NPL];
+                double pv, ov;
                 const double *cx = sx + ri, *cy = sy + ri, *cz = sz + ri;
                 const double2 *cxy = (const double2 *)sx + ri, *czl = (const double2 *)sz + ri;
-#pragma unroll
-                for (int m = 0; m < NPL; m++) {
+                auto pair_reads = [&](int m) __attribute__((always_inline)) {
                     if (MIXED) {
                         const double2 pa = cxy[dl[m]], pb = cxy[-dl[m]];
                         const double2 za = czl[dl[m]], zb = czl[-dl[m]];
@@ -325,98 +391,96 @@ __global__ __launch_bounds__(BLK) void tile_sweep_kernel(SweepArgs a, int first_
                         ax[m] = cx[dl[m]]; ay[m] = cy[dl[m]]; az[m] = cz[dl[m]];
                         bx[m] = cx[-dl[m]]; by[m] = cy[-dl[m]]; bz[m] = cz[-dl[m]];
                     }
-                }
-                const double px = prop[pq], py = prop[PS + pq], pz = prop[2 * PS + pq];
-                const double thr = prop[3 * PS + pq];
-                const double ox = sx[ZS * ri], oy = sy[ZS * ri], oz = sz[ZS * ri];
-                const double Li = MIXED ? sl[2 * ri] : rep.L0;
-                asm volatile("" ::: "memory");
+                };
+                auto site_reads = [&]() __attribute__((always_inline)) {
+                    pv = prop[4 * pq + comp];
+                    ov = own[ZS * ri];
+                };
+                // The reads run AHEAD pairs ahead of the sums: a wave's wait
+                // names at most 15 outstanding LDS reads, so with all of a
+                // step's reads issued at once the first sums waited for half of
+                // them (64^3: 10.51 -> 10.35 ms per 50 sweeps)
+                constexpr int AHEAD = NPL < 3 ? NPL : 3;
+#pragma unroll
+                for (int m = 0; m < AHEAD; m++) pair_reads(m);
+                if (NPL == AHEAD) site_reads();
 #pragma unroll
                 for (int m = 0; m < NPL; m++) {
-                    const double ux = ax[m] + bx[m], uy = ay[m] + by[m], uz = az[m] + bz[m];
+                    asm volatile("" ::: "memory");
                     double mx, my, mz;
                     if (MIXED) {
                         mx = la[m] * ax[m] + lb[m] * bx[m];
                         my = la[m] * ay[m] + lb[m] * by[m];
                         mz = la[m] * az[m] + lb[m] * bz[m];
+                        if (m == 0) {
+                            gx_ = nnf * (ax[0] + bx[0]); gy_ = nnf * (ay[0] + by[0]); gz_ = nnf * (az[0] + bz[0]);
+                        }
                     } else {
-                        mx = ux; my = uy; mz = uz;
+                        mx = ax[m] + bx[m]; my = ay[m] + by[m]; mz = az[m] + bz[m];
                     }
                     const double s = nx[m] * mx + ny[m] * my + nz[m] * mz;
                     // the first pair starts the sums (no adds of +0.0); each
                     // component is two dependent FMAs
-                    if constexpr (TN) {
-                        if (m == 0) {
-                            hx_ = fma(s, t3.x[m], wn0 * mx);
-                            hy_ = fma(s, t3.y[m], wn0 * my);
-                            hz_ = fma(s, t3.z[m], wn0 * mz);
-                            if (MIXED) { gx_ = nnf * ux; gy_ = nnf * uy; gz_ = nnf * uz; }
-                        } else {
-                            hx_ = fma(s, t3.x[m], fma(w[m], mx, hx_));
-                            hy_ = fma(s, t3.y[m], fma(w[m], my, hy_));
-                            hz_ = fma(s, t3.z[m], fma(w[m], mz, hz_));
-                        }
-                        continue;
-                    }
-                    const double ts = w3[m] * s;
-                    if (m == 0) {
-                        hx_ = fma(ts, nx[m], wn0 * mx);
-                        hy_ = fma(ts, ny[m], wn0 * my);
-                        hz_ = fma(ts, nz[m], wn0 * mz);
-                        if (MIXED) { gx_ = nnf * ux; gy_ = nnf * uy; gz_ = nnf * uz; }
-                    } else {
-                        hx_ = fma(ts, nx[m], fma(w[m], mx, hx_));
-                        hy_ = fma(ts, ny[m], fma(w[m], my, hy_));
-                        hz_ = fma(ts, nz[m], fma(w[m], mz, hz_));
-                    }
+                    double tx, ty, tz, f;
+                    if constexpr (TN) { tx = t3.x[m]; ty = t3.y[m]; tz = t3.z[m]; f = s; }
+                    else { tx = nx[m]; ty = ny[m]; tz = nz[m]; f = w3[m] * s; }
+                    hx_ = fma(f, tx, m == 0 ? (MIXED ? w[m] * mx : fma(w[m], mx, E0)) : fma(w[m], mx, hx_));
+                    hy_ = fma(f, ty, m == 0 ? (MIXED ? w[m] * my : fma(w[m], my, E1)) : fma(w[m], my, hy_));
+                    hz_ = fma(f, tz, m == 0 ? (MIXED ? w[m] * mz : fma(w[m], mz, E2)) : fma(w[m], mz, hz_));
+                    asm volatile("" : "+v"(hx_), "+v"(hy_), "+v"(hz_) : : "memory");
+                    if (m + AHEAD < NPL) pair_reads(m + AHEAD);
+                    if (m + AHEAD + 1 == NPL) site_reads();
                 }
-                const double coef = MIXED ? Li : Li * rep.L0;
-                const double dx = px - ox, dy = py - oy, dz = pz - oz;
-                double partial = coef * (dx * hx_ + dy * hy_ + dz * hz_);
-                if (MIXED) partial -= J * (dx * gx_ + dy * gy_ + dz * gz_);
-                partial = group_sum_dpp<G>(partial);
-                double dE = partial + (dx * E0 + dy * E1 + dz * E2);
-                if (K > 0.0) dE += -K * (fabs(px) - fabs(ox) + fabs(py) - fabs(oy));
-                const bool acc = dE < thr;
-                if (part == 0 && Li != 0.0) {
-                    if (acc) {
-                        sx[ZS * ri] = px; sy[ZS * ri] = py; sz[ZS * ri] = pz;
-                        nacc++;
-                    } else nrej++;
+                if (MIXED) {
+                    const double Li = lane_bcast<3, G>(ov);
+                    hx_ = fma(Li, hx_, fma(-J, gx_, E0)); hy_ = fma(Li, hy_, fma(-J, gy_, E1));
+                    hz_ = fma(Li, hz_, fma(-J, gz_, E2));
+                }
+                const double d = pv - ov;
+                double dE = lane_bcast<0, G>(d) * hx_ + lane_bcast<1, G>(d) * hy_ + lane_bcast<2, G>(d) * hz_;
+                if (K > 0.0) {   // (kept a branch: three instructions in every step otherwise)
+                    asm volatile("" ::: "memory");
+                    dE -= Kp * (fabs(pv) - fabs(ov));
+                }
+                dE = group_sum_dpp<G>(dE);
+                // (the fence keeps the exchange above the branch, where lane 3 is on)
+                double thr = lane_bcast<3, G>(pv);
+                asm volatile("" : "+v"(thr));
+                nvis++;
+                if (writer && dE < thr) {
+                    own[ZS * ri] = pv;
+                    nacc++;
                 }
             }
-            if (flag) __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(e) & kStepBarrier) __syncthreads();
             e = e_next;
-            flag = flag_next;
         }
     }
 
-    // ---- write the tile back ----
-    double4 *out = a.lat + rep.base;
-    for (int i = tid; i < ntile; i += BLK) {
-        int lz = i % sh.tz, q = i / sh.tz;
-        int ly = q % sh.ty, lx = q / sh.ty;
-        int ri = ((lx + hx) * RY + (ly + hy)) * RZs + (lz + hz);
-        double4 v;
-        v.x = sx[ZS * ri]; v.y = sy[ZS * ri]; v.z = sz[ZS * ri];
-        v.w = MIXED ? sl[2 * ri] : rep.L0;
-        out[tile_base + ((long long)lx * rep.Y + ly) * rep.Z + lz] = v;
+    // ---- counters: this tile's own slot (one workgroup per tile per launch;
+    // adds without a return value, before the tile's stores, so that nothing
+    // waits for the old count or for the stores) ----
+    if (part == 0 && nvis && writer) {
+        if (nacc) atomicAdd(&s_cnt[0], nacc);
+        atomicAdd(&s_cnt[1], nvis - nacc);
     }
-    // ---- counters: this tile's own slot (one workgroup per tile per launch) ----
-    unsigned long long ca = nacc, cr = nrej;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        ca += __shfl_xor(ca, o, 64);
-        cr += __shfl_xor(cr, o, 64);
-    }
-    __shared__ unsigned long long s_cnt[2 * (BLK / 64)];
-    if ((tid & 63) == 0) { s_cnt[2 * (tid >> 6)] = ca; s_cnt[2 * (tid >> 6) + 1] = cr; }
     __syncthreads();
-    if (tid == 0) {
-        unsigned long long A_ = 0, R_ = 0;
-        for (int w_ = 0; w_ < BLK / 64; w_++) { A_ += s_cnt[2 * w_]; R_ += s_cnt[2 * w_ + 1]; }
-        a.counters[2 * (first_tile + t)] += A_;
-        a.counters[2 * (first_tile + t) + 1] += R_;
+    if (tid < 2) atomicAdd(a.counters + 2 * (first_tile + t) + tid, (unsigned long long)s_cnt[tid]);
+
+    // ---- write the tile back ----
+    double4 *out = a.lat + tile.base;
+    {
+        const int trows = ty * tz, tper = trows < BLK ? BLK / trows : 1;
+        for (int q = tid; q < (trows < BLK ? tper * trows : trows); q += BLK) {
+            const int px = q / trows, k = q - px * trows, ly = k / tz, lz = k - ly * tz;
+            for (int lx = px; lx < tx; lx += tper) {
+                const int ri = ((lx + hx) * RY + (ly + hy)) * RZs + (lz + hz);
+                double4 o;
+                o.x = sx[ZS * ri]; o.y = sy[ZS * ri]; o.z = sz[ZS * ri];
+                o.w = MIXED ? sl[2 * ri] : rep.L0;
+                out[tile_base + ((long long)lx * tile.Y + ly) * tile.Z + lz] = o;
+            }
+        }
     }
 }
 
