@@ -2,9 +2,11 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -94,7 +96,10 @@ struct sn_ctx {
     std::vector<std::vector<int32_t>> torus_order, torus_cstart;   // per replica: sites by colour, colour starts
     int torus_ncol = 0;                                             // colours per sweep (shorter colourings padded)
     int torus_G = 0, torus_NPL = 0, torus_blk = 0, torus_ms = 0, torus_mc = 0, torus_pc = 0;
-    int *d_torus_sites = nullptr, *d_torus_off = nullptr, *d_torus_cs = nullptr;
+    int *d_torus_box_of = nullptr, *d_torus_sites = nullptr, *d_torus_entries = nullptr, *d_torus_chunks = nullptr;
+    TorusBox *d_torus_boxes = nullptr;
+    unsigned short *d_torus_near = nullptr;
+    int torus_max_chunks = 0;
     unsigned long long *d_rep_counters = nullptr;   // 2 per replica (torus sweeps)
     bool can_sweep = false;
     std::string sweep_err;
@@ -342,8 +347,8 @@ constexpr int kTorusMaxIndex = 128;
 
 static size_t torus_lds(const sn_ctx *c, bool mixed)
 {
-    return (size_t)((mixed ? 4 : 3) * c->torus_ms + 4 * c->torus_pc) * sizeof(double) +
-           (size_t)c->torus_ms * sizeof(int);
+    return (size_t)((((mixed ? 4 : 3) * c->torus_ms + 1) & ~1) + 4 * c->torus_pc) * sizeof(double) +
+           (size_t)2 * (c->torus_max_chunks + 1) * sizeof(int);
 }
 
 // lanes per site, pairs per lane and threads for npairs pairs and colours of
@@ -426,23 +431,12 @@ static int setup_torus(sn_ctx *c)
     const bool greedy = gcost >= 0 && (lcost < 0 || gcost < lcost);
     c->torus_order = greedy ? go : lo;
     c->torus_cstart = greedy ? gs : ls;
-    // no empty colour before a replica's last site: the kernel's lookahead
-    // takes an empty colour for the end of the replica's sites
+    // no empty colour before a replica's last site
     for (auto &st_ : c->torus_cstart) st_.erase(std::unique(st_.begin(), st_.end()), st_.end());
     c->torus_ncol = 0;
     for (const auto &st : c->torus_cstart) c->torus_ncol = std::max(c->torus_ncol, (int)st.size() - 1);
-    std::vector<int> sites, off, cs;
-    for (int r = 0; r < c->R; r++) {
-        const ReplicaGeom &g = c->geom[r];
-        off.push_back((int)sites.size());
-        for (int32_t si : c->torus_order[r]) {   // packed coordinates x | y << 10 | z << 20
-            const int z = si % g.Z, xy = si / g.Z, y = xy % g.Y, x = xy / g.Y;
-            sites.push_back(x | (y << 10) | (z << 20));
-        }
-        std::vector<int32_t> &st_ = c->torus_cstart[r];
+    for (auto &st_ : c->torus_cstart)
         while ((int)st_.size() < c->torus_ncol + 1) st_.push_back(st_.back());   // empty colours
-        cs.insert(cs.end(), st_.begin(), st_.end());
-    }
     c->torus_mc = max_class(c->torus_cstart);
     int G, NPL, blk;
     if (!torus_shape(np, c->torus_mc, greedy, G, NPL, blk))
@@ -464,19 +458,78 @@ static int setup_torus(sn_ctx *c)
     // for (at most the largest replica, at least the largest colour)
     const long long room = (150LL * 1024 / (long long)sizeof(double) - 4LL * c->torus_ms - c->torus_ms / 2) / 4;
     c->torus_pc = (int)std::max<long long>(c->torus_mc, std::min<long long>(room, c->torus_ms));
-    const size_t lds = torus_lds(c, true);
-    if (lds > 150 * 1024)
+    // tables of each box size: the sites by colour, the rounds' entries and
+    // neighbours, the runs of colours whose proposals are drawn together
+    const int NG = blk / G;
+    const std::vector<Offset> pairs = neighbour_pairs(c->rc, c->two_d);
+    std::vector<TorusBox> boxes;
+    std::vector<int> box_of, sites, entries, chunks;
+    std::vector<unsigned short> near;
+    std::map<std::array<int, 3>, int> known;
+    for (int r = 0; r < c->R; r++) {
+        const ReplicaGeom &g = c->geom[r];
+        const auto at = known.emplace(std::array<int, 3>{g.X, g.Y, g.Z}, (int)boxes.size());
+        box_of.push_back(at.first->second);
+        if (!at.second) continue;
+        const std::vector<int32_t> &o = c->torus_order[r], &cst = c->torus_cstart[r];
+        TorusBox b{};
+        b.sites_off = (int)sites.size();
+        b.entry_off = (int)entries.size();
+        b.chunk_off = (int)chunks.size();
+        b.near_off = (long long)near.size();
+        sites.insert(sites.end(), o.begin(), o.end());
+        const int ncol = (int)cst.size() - 1;
+        int p0 = 0;   // first site of the run of colours
+        for (int k = 0; k < ncol; k++) {
+            if (k == 0 || cst[k + 1] - p0 > c->torus_pc) {
+                p0 = cst[k];
+                chunks.push_back(b.nrounds);
+                chunks.push_back(p0);
+                b.nchunks++;
+            }
+            for (int b0 = cst[k]; b0 < cst[k + 1]; b0 += NG, b.nrounds++) {
+                const bool last = b0 + NG >= cst[k + 1];
+                for (int q = 0; q < NG; q++) {
+                    const bool idle = b0 + q >= cst[k + 1];
+                    const int si = idle ? o[0] : o[b0 + q];
+                    entries.push_back(torus_entry(si, idle ? 0 : b0 + q - p0, last, idle));
+                    const int z = si % g.Z, y = si / g.Z % g.Y, x = si / (g.Z * g.Y);
+                    auto at8 = [&](int a, int bb, int cc) {
+                        a = (a + g.X) % g.X; bb = (bb + g.Y) % g.Y; cc = (cc + g.Z) % g.Z;
+                        return (unsigned short)(8 * ((a * g.Y + bb) * g.Z + cc));
+                    };
+                    for (int part = 0; part < G; part++)
+                        for (int m = 0; m < NPL; m++) {
+                            Offset d{0, 0, 0, 0};   // a padded pair: the site itself, with no weight
+                            if (part + m * G < np) d = pairs[part + m * G];
+                            near.push_back(at8(x + d.dx, y + d.dy, z + d.dz));
+                            near.push_back(at8(x - d.dx, y - d.dy, z - d.dz));
+                        }
+                }
+            }
+        }
+        chunks.push_back(b.nrounds);
+        chunks.push_back(cst[ncol]);
+        c->torus_max_chunks = std::max(c->torus_max_chunks, b.nchunks);
+        boxes.push_back(b);
+    }
+    // (four arrays, proposals and an int per site: what a replica may take)
+    if ((size_t)4 * (c->torus_ms + c->torus_pc) * sizeof(double) + (size_t)c->torus_ms * sizeof(int) > 150 * 1024 ||
+        c->torus_ms > kTorusMaxSites)
         return fail(c, SN_ERR_UNSUPPORTED, "whole-lattice sweep: a replica does not fit in LDS (" +
                                                std::to_string(c->torus_ms) + " sites)");
     int st;
     for (int m = 0; m < 2; m++) {
         const void *f = (const void *)pick_torus(G, NPL, m == 1, blk);
         if (!f) return fail(c, SN_ERR_UNSUPPORTED, "whole-lattice sweep: no kernel for this cutoff");
-        HIPCHK(c, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        HIPCHK(c, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)torus_lds(c, true)));
     }
+    if ((st = upload(c, &c->d_torus_box_of, box_of))) return st;
+    if ((st = upload(c, &c->d_torus_boxes, boxes))) return st;
     if ((st = upload(c, &c->d_torus_sites, sites))) return st;
-    if ((st = upload(c, &c->d_torus_off, off))) return st;
-    if ((st = upload(c, &c->d_torus_cs, cs))) return st;
+    if ((st = upload(c, &c->d_torus_entries, entries))) return st;
+    if ((st = upload(c, &c->d_torus_near, near))) return st;
+    if ((st = upload(c, &c->d_torus_chunks, chunks))) return st;
     std::vector<unsigned long long> z(2 * c->R, 0ull);
     if ((st = upload(c, &c->d_rep_counters, z))) return st;
     c->torus = true;
@@ -848,8 +901,8 @@ int sn_destroy(sn_ctx *c)
                     c->d_field_steps, c->d_tile_coord, c->d_gsteps, c->d_pairs,
                     c->d_offs, c->d_sweep,
                     c->d_counters, c->d_partials, c->d_result, c->d_radial, c->d_radial_bins,
-                    c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_sites,
-                    c->d_torus_off, c->d_torus_cs, c->d_rep_counters, c->d_stage};
+                    c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
+                    c->d_torus_sites, c->d_torus_entries, c->d_torus_near, c->d_torus_chunks, c->d_rep_counters, c->d_stage};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_result) (void)hipHostFree(c->h_result);
@@ -1092,9 +1145,10 @@ static int launch_torus(sn_ctx *c, int nsw, std::vector<hipEvent_t> *events)
 {
     const bool mixed = any_mixed(c);
     TorusArgs t;
-    t.lat = c->d_lat; t.reps = c->d_reps; t.pairs = c->d_pairs; t.npairs = c->npairs;
-    t.sites = c->d_torus_sites; t.site_off = c->d_torus_off; t.col_start = c->d_torus_cs;
-    t.ncol = c->torus_ncol; t.sweep_ctr = c->d_sweep; t.counters = c->d_rep_counters;
+    t.lat = c->d_lat; t.reps = c->d_reps; t.pairs = c->d_pairs;
+    t.box_of = c->d_torus_box_of; t.boxes = c->d_torus_boxes; t.sites = c->d_torus_sites;
+    t.entries = c->d_torus_entries; t.nears = c->d_torus_near; t.chunks = c->d_torus_chunks;
+    t.sweep_ctr = c->d_sweep; t.counters = c->d_rep_counters;
     t.max_sites = c->torus_ms; t.prop_cap = c->torus_pc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (events && (event_pair(c, events, &e0, &e1) || hipEventRecord(e0, c->stream) != hipSuccess))

@@ -6,8 +6,10 @@
 // sublattice that holds the replica's box vectors and whose shortest vector is
 // longer than DipoleCutOff, so the sites of one colour are more than rc apart
 // through the periodic boundary and update together; colours follow one
-// another with a workgroup barrier.  Neighbour indices wrap periodically on
-// the fly (the reference's % X wrap, src/starrynight-montecarlo-core.c:97).
+// another with a workgroup barrier.  The neighbours' LDS addresses (periodic
+// wrap, the reference's % X, src/starrynight-montecarlo-core.c:97) come from a
+// table of the replica's box, streamed from L2 two rounds ahead: forming them in
+// the round took 66 of its instructions (25 x 25), after the barrier.
 // Per site the arithmetic is the tile kernels': G lanes share a site, each
 // lane takes NPL of the +-r pairs, one scalar per lane is reduced over the
 // group, and the Metropolis threshold and proposal come from the same
@@ -17,15 +19,25 @@
 
 namespace sn {
 
+// One box size: where its tables start.
+struct TorusBox {
+    int sites_off;             // sites by colour (linear index), N of them
+    int entry_off, nrounds;    // NG step_entry's per round; rounds of one sweep
+    int chunk_off, nchunks;    // first round and first site of each run of proposals (nchunks + 1 of both)
+    int pad;
+    long long near_off;        // 2 NPL shorts per lane and round
+};
+
 struct TorusArgs {
     double4 *lat;
     const RepDev *reps;
-    const PairDev *pairs;
-    int npairs;
-    const int *sites;          // per replica (at site_off[r]): sites by colour, packed x | y << 10 | z << 20
-    const int *site_off;       // R entries
-    const int *col_start;      // per replica: ncol + 1 colour starts (at r * (ncol + 1))
-    int ncol;
+    const PairDev *pairs;      // padded with zero pairs to kPairSlots
+    const int *box_of;         // R entries
+    const TorusBox *boxes;
+    const int *sites;          // per box (sites_off)
+    const int *entries;        // per box (entry_off): site | slot << 13 by group, flags as step_entry
+    const unsigned short *nears;   // per box (near_off): 8 x site index of the lane's neighbours, + and - of each pair
+    const int *chunks;         // per box (chunk_off)
     const unsigned *sweep_ctr;
     unsigned long long *counters;  // 2 per replica: accepted, rejected (accumulated)
     int max_sites;             // stride of the staged arrays
@@ -33,214 +45,204 @@ struct TorusArgs {
                                // runs of at most this many sites
 };
 
-// (c + d) mod L for 0 <= c < L and |d| < L, without branches: of c + d and
-// c + d + s (s = -L for d >= 0, +L for d < 0) one lies in [0, L) and the other
-// is negative or >= L, so as unsigned values the smaller one is the answer.
-__device__ __forceinline__ int wrap_pm(int t, int s) { return (int)min((unsigned)t, (unsigned)(t + s)); }
+// Entry of a lane group: site and proposal slot have 13 bits each (a replica
+// of at most kTorusMaxSites fits in LDS).
+constexpr int kTorusMaxSites = 8191;
+__host__ __device__ inline int torus_entry(int site, int slot, bool last, bool idle)
+{
+    return site | (slot << 13) | (last ? kStepBarrier : 0) | (idle ? kStepIdle : 0);
+}
 
 template <int G, int NPL, bool MIXED, int BLK>
 __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nsweeps)
 {
-    extern __shared__ double smem[];
+    static_assert(G * NPL <= kPairSlots, "the pair table covers every lane's slots");
+    extern __shared__ __align__(16) double smem[];
     const int tid = threadIdx.x, r = blockIdx.x;
     const RepDev rep = t.reps[r];
-    const int X = rep.X, Y = rep.Y, Z = rep.Z, N = X * Y * Z, YZ = Y * Z;   // N < 2^24 (LDS)
+    const TorusBox box = t.boxes[t.box_of[r]];
+    const int N = rep.X * rep.Y * rep.Z;
     const int MS = t.max_sites, PS = t.prop_cap;
-    double *sx = smem, *sy = sx + MS, *sz = sy + MS, *sl = sz + MS;
-    double *prop = MIXED ? sl + MS : sl;    // 4 x PS: px, py, pz, threshold of the colour's sites
-    int *sites = (int *)(prop + 4 * PS);    // the replica's site table (MS ints)
-    const int *cs = t.col_start + r * (t.ncol + 1);   // colour starts (uniform: scalar loads)
-    const int ncol = t.ncol;
+    // as the tile sweep: x, y and z arrays, or (x, y) and (z, L) pairs
+    constexpr int ZS = MIXED ? 2 : 1;
+    double *sx = smem;
+    double *sy = MIXED ? sx + 1 : sx + MS;
+    double *sz = sx + 2 * MS;
+    double *prop = sx + (((MIXED ? 4 : 3) * MS + 1) & ~1);   // px, py, pz and threshold of slot k at prop[4 k]
+    int *s_chunk = (int *)(prop + 4 * PS);
     double4 *lat = t.lat + rep.base;
 
-    // ---- the whole replica and its site table into LDS ----
-    const int *gsites = t.sites + t.site_off[r];
+    // ---- the whole replica into LDS ----
     for (int i = tid; i < N; i += BLK) {
         const double4 v = lat[i];
-        sx[i] = v.x; sy[i] = v.y; sz[i] = v.z;
-        if (MIXED) sl[i] = v.w;
-        sites[i] = gsites[i];
+        if (MIXED) {
+            ((double2 *)sx)[i] = make_double2(v.x, v.y);
+            ((double2 *)sz)[i] = make_double2(v.z, v.w);
+        } else {
+            sx[i] = v.x; sy[i] = v.y; sz[i] = v.z;
+        }
     }
+    for (int i = tid; i < 2 * (box.nchunks + 1); i += BLK) s_chunk[i] = t.chunks[box.chunk_off + i];
 
     // ---- this lane's share of the +-r pairs ----
     const int part = tid % G, group = tid / G;
     constexpr int NG = BLK / G;
-    int pdx[NPL], pdy[NPL], pdz[NPL], swx[NPL], swy[NPL], swz[NPL];   // offsets, wrap steps of +d
-    double nx[NPL], ny[NPL], nz[NPL], w[NPL], w3[NPL];
+    double nx[NPL], ny[NPL], nz[NPL], w[NPL], w3[NPL], nnf = 0.0;
 #pragma unroll
     for (int m = 0; m < NPL; m++) {
-        const int j = part + m * G;
-        if (j < t.npairs) {
-            const PairDev p = t.pairs[j];
-            pdx[m] = p.dx; pdy[m] = p.dy; pdz[m] = p.dz;
-            swx[m] = p.dx >= 0 ? -X : X; swy[m] = p.dy >= 0 ? -Y : Y; swz[m] = p.dz >= 0 ? -Z : Z;
-            nx[m] = p.nx; ny[m] = p.ny; nz[m] = p.nz; w[m] = p.w; w3[m] = -3.0 * p.w;
-        } else {
-            pdx[m] = 0; pdy[m] = 0; pdz[m] = 0; swx[m] = -X; swy[m] = -Y; swz[m] = -Z;
-            nx[m] = 0.0; ny[m] = 0.0; nz[m] = 0.0; w[m] = 0.0; w3[m] = 0.0;
-        }
+        const PairDev p = t.pairs[part + m * G];
+        nx[m] = p.nx; ny[m] = p.ny; nz[m] = p.nz; w[m] = p.w; w3[m] = -3.0 * p.w;
+        // nearest-neighbour pairs come first in the table, so they sit in slot 0
+        if (m == 0) nnf = p.nn ? 1.0 : 0.0;
     }
-    // nearest-neighbour pairs come first in the table, so they sit in slot 0
-    const double nnf = (part < t.npairs && t.pairs[part].nn) ? 1.0 : 0.0;
     const double rbeta = 1.0 / rep.beta;
-    const double J = rep.J, K = rep.K, E0 = rep.E[0], E1 = rep.E[1], E2 = rep.E[2];
-    // uniform lengths: the cage-strain sum rides on the nearest-neighbour weight
-    const double wn0 = (!MIXED && nnf != 0.0 && rep.L0 != 0.0) ? w[0] - J / (rep.L0 * rep.L0) : w[0];
-    unsigned nacc = 0, nrej = 0;
-    __syncthreads();
-
-    // One round: the group's site of colour k starting at site b (its entry
-    // q = b + group, active while q < the colour's end).  The site table never
-    // changes, so with LOOKAHEAD a round's site and its neighbours' indices
-    // are found during the previous round, and after a colour's barrier a
-    // round goes straight to its LDS reads.  Measured (site-updates/s, 64 or
-    // 256 replicas): +20-26% at 4 pairs a lane (12^3 at DipoleCutOff 1-3, 2D
-    // 30 x 30 at 2, 4, 5), -3 to -5% at 1-2 pairs a lane (25 x 25, 16 x 16 x 8
-    // at DipoleCutOff 3, 12^3 at 4), which find their site after the barrier.
-    constexpr bool LOOKAHEAD = NPL >= 4;
-    struct Round {
-        bool act;
-        int si, pq, ia[NPL], ib[NPL];
-    };
-    // the site entry of the round at (k, b) (the site table never changes)
-    auto entry = [&](int k, int b) __attribute__((always_inline)) {
-        const int q = b + group;
-        return q < cs[k + 1] ? sites[q] : -1;
-    };
-    auto prepare = [&](int pk, int pq) __attribute__((always_inline)) {
-        Round R;
-        R.act = pk >= 0;
-        const int x = pk & 1023, y = (pk >> 10) & 1023, z = (pk >> 20) & 1023;
-        R.si = __umul24(x, YZ) + __umul24(y, Z) + z;
+    // the field term, the factors of uniform lengths and a site's own
+    // components: see the tile sweep
+    const double J = rep.J, K = rep.K;
+    const double E0 = part == 0 ? rep.E[0] : 0.0, E1 = part == 0 ? rep.E[1] : 0.0, E2 = part == 0 ? rep.E[2] : 0.0;
+    if constexpr (!MIXED) {
+        const double LL = rep.L0 * rep.L0;
 #pragma unroll
-        for (int m = 0; m < NPL; m++) {
-            // periodic wrap of x +- dx etc. (|d| <= rc < length; -d wraps
-            // the other way, so its step is -s)
-            const int xa = wrap_pm(x + pdx[m], swx[m]), xb = wrap_pm(x - pdx[m], -swx[m]);
-            const int ya = wrap_pm(y + pdy[m], swy[m]), yb = wrap_pm(y - pdy[m], -swy[m]);
-            const int za = wrap_pm(z + pdz[m], swz[m]), zb = wrap_pm(z - pdz[m], -swz[m]);
-            R.ia[m] = __umul24(xa, YZ) + __umul24(ya, Z) + za;
-            R.ib[m] = __umul24(xb, YZ) + __umul24(yb, Z) + zb;
-        }
-        R.pq = pq;
-        return R;
+        for (int m = 0; m < NPL; m++) { w[m] *= LL; w3[m] *= LL; }
+        w[0] -= nnf * J;
+    }
+    const int comp = part & 3;
+    double *own = MIXED ? sx + (comp >> 1) * 2 * MS + (comp & 1) : sx + (comp < 3 ? comp : 2) * MS;
+    const double Kp = part < 2 ? K : 0.0;
+    const bool writer = part < 3 && (MIXED || rep.L0 != 0.0);   // vacancies never move and are not counted
+    unsigned nacc = 0, nvis = 0;   // accepted (on a group's first lane), visited
+    __shared__ unsigned s_cnt[2];
+    if (tid < 2) s_cnt[tid] = 0;
+
+    // ---- the round tables, two rounds ahead of their use ----
+    struct Near {
+        unsigned ab[NPL];   // 8 x site of the pair's + neighbour, - neighbour << 16
     };
+    const int *entries = t.entries + box.entry_off + group;
+    const Near *nears = (const Near *)(t.nears + box.near_off) + tid;
+    int e0, e1, e2;
+    Near n0, n1, n2;
+    int ahead = 0;   // the round loaded next (the sweep's rounds repeat)
+    auto fetch = [&](int &e, Near &n) __attribute__((always_inline)) {
+        e = entries[ahead * NG];
+        n = nears[(long long)ahead * BLK];
+        ahead = ahead + 1 < box.nrounds ? ahead + 1 : 0;
+    };
+    fetch(e0, n0);
+    fetch(e1, n1);
+    __syncthreads();
 
     for (int s = 0; s < nsweeps; s++) {
         const unsigned sweep = t.sweep_ctr[r] + (unsigned)s;
-        for (int k0 = 0; k0 < ncol;) {
-            // ---- proposals of a run of colours [k0, k1) holding at most PS sites ----
-            int k1 = k0 + 1;
-            while (k1 < ncol && cs[k1 + 1] - cs[k0] <= PS) k1++;
-            const int p0 = cs[k0];
-            for (int i = tid; i < cs[k1] - p0; i += BLK) {
-                double px, py, pz, u;
-                const int pk = sites[p0 + i];
-                const int si = __umul24(pk & 1023, YZ) + __umul24((pk >> 10) & 1023, Z) + (pk >> 20);
-                counter_draw(rep.seed, (uint32_t)r, sweep, (unsigned)si, rep.constrain_to_x, px, py, pz, u);
-                prop[i] = px;
-                prop[PS + i] = py;
-                prop[2 * PS + i] = pz;
-                prop[3 * PS + i] = metropolis_threshold(u, rep.beta, rbeta);
+        for (int ch = 0; ch < box.nchunks; ch++) {
+            // ---- proposals of a run of colours, two sites per lane at a time ----
+            const int p0 = s_chunk[2 * ch + 1], np = s_chunk[2 * ch + 3] - p0;
+            for (int i = tid; i < np; i += 2 * BLK) {
+                const bool two = i + BLK < np;
+                const uint32_t site[2] = {(uint32_t)t.sites[box.sites_off + p0 + i],
+                                          (uint32_t)t.sites[box.sites_off + p0 + (two ? i + BLK : i)]};
+                double px[2], py[2], pz[2], u[2];
+                counter_draws<2>(rep.seed, (uint32_t)r, sweep, site, rep.constrain_to_x, px, py, pz, u);
+#pragma unroll
+                for (int q = 0; q < 2; q++)
+                    if (q == 0 || two) {
+                        ((double2 *)prop)[2 * (i + q * BLK)] = make_double2(px[q], py[q]);
+                        ((double2 *)prop)[2 * (i + q * BLK) + 1] =
+                            make_double2(pz[q], metropolis_threshold(u[q], rep.beta, rbeta));
+                    }
             }
+            const int r0 = __builtin_amdgcn_readfirstlane(s_chunk[2 * ch]);
+            const int r1 = __builtin_amdgcn_readfirstlane(s_chunk[2 * ch + 2]);
             __syncthreads();
-            // ---- the run's colours, NG sites at a time (a colour's sites are
-            // independent of each other); a barrier ends each colour ----
-            // (empty colours, the padding of replicas with fewer colours, come
-            // after all of a replica's sites: a lookahead that reaches one
-            // finds no site, and neither do the colours after it)
-            Round cur;
-            if constexpr (LOOKAHEAD) cur = prepare(entry(k0, p0), group);
-            for (int k = k0; k < k1; k++) {
-                const int c1 = cs[k + 1];
-                for (int b0 = cs[k]; b0 < c1; b0 += NG) {
-                    const bool last = b0 + NG >= c1;           // the colour's last round
-                    const int kn = last ? k + 1 : k, bn = last ? c1 : b0 + NG;
-                    int pk_next = -1;
-                    if constexpr (LOOKAHEAD) pk_next = kn < k1 ? entry(kn, bn) : -1;
-                    else cur = prepare(entry(k, b0), b0 + group - p0);
-                    if (cur.act) {   // whole groups (DPP rows) are active or not
-                        double hx_, hy_, hz_, gx_ = 0.0, gy_ = 0.0, gz_ = 0.0;
-                        double ax[NPL], ay[NPL], az[NPL], bx[NPL], by[NPL], bz[NPL], la[NPL], lb[NPL];
+            // ---- the run's rounds: every group decides one site; a colour's
+            // last round ends with the barrier (before it, rounds of a colour
+            // are independent of each other) ----
+            for (int rd = r0; rd < r1; rd++) {
+                fetch(e2, n2);
+                if (e0 >= 0) {   // whole groups are active or not
+                    const int si = e0 & 8191, pq = (e0 >> 13) & 8191;
+                    double hx_, hy_, hz_, gx_, gy_, gz_;
+                    double ax[NPL], ay[NPL], az[NPL], bx[NPL], by[NPL], bz[NPL], la[NPL], lb[NPL];
 #pragma unroll
-                        for (int m = 0; m < NPL; m++) {
-                            const int ia = cur.ia[m], ib = cur.ib[m];
-                            ax[m] = sx[ia]; ay[m] = sy[ia]; az[m] = sz[ia];
-                            bx[m] = sx[ib]; by[m] = sy[ib]; bz[m] = sz[ib];
-                            if (MIXED) { la[m] = sl[ia]; lb[m] = sl[ib]; }
-                        }
-                        const int pq = cur.pq, si = cur.si;
-                        const double px = prop[pq], py = prop[PS + pq], pz = prop[2 * PS + pq];
-                        const double thr = prop[3 * PS + pq];
-                        const double ox = sx[si], oy = sy[si], oz = sz[si];
-                        const double Li = MIXED ? sl[si] : rep.L0;
-#pragma unroll
-                        for (int m = 0; m < NPL; m++) {
-                            const double ux = ax[m] + bx[m], uy = ay[m] + by[m], uz = az[m] + bz[m];
-                            double mx, my, mz;
-                            if (MIXED) {
-                                mx = la[m] * ax[m] + lb[m] * bx[m];
-                                my = la[m] * ay[m] + lb[m] * by[m];
-                                mz = la[m] * az[m] + lb[m] * bz[m];
-                            } else {
-                                mx = ux; my = uy; mz = uz;
-                            }
-                            const double sdot = nx[m] * mx + ny[m] * my + nz[m] * mz;
-                            const double ts = w3[m] * sdot;
-                            if (m == 0) {
-                                hx_ = fma(ts, nx[m], wn0 * mx);
-                                hy_ = fma(ts, ny[m], wn0 * my);
-                                hz_ = fma(ts, nz[m], wn0 * mz);
-                                if (MIXED) { gx_ = nnf * ux; gy_ = nnf * uy; gz_ = nnf * uz; }
-                            } else {
-                                hx_ = fma(ts, nx[m], fma(w[m], mx, hx_));
-                                hy_ = fma(ts, ny[m], fma(w[m], my, hy_));
-                                hz_ = fma(ts, nz[m], fma(w[m], mz, hz_));
-                            }
-                        }
-                        const double coef = MIXED ? Li : Li * rep.L0;
-                        const double dx = px - ox, dy = py - oy, dz = pz - oz;
-                        double partial = coef * (dx * hx_ + dy * hy_ + dz * hz_);
-                        if (MIXED) partial -= J * (dx * gx_ + dy * gy_ + dz * gz_);
-                        partial = group_sum_dpp<G>(partial);
-                        double dE = partial + (dx * E0 + dy * E1 + dz * E2);
-                        if (K > 0.0) dE += -K * (fabs(px) - fabs(ox) + fabs(py) - fabs(oy));
-                        if (part == 0 && Li != 0.0) {   // vacancies never move
-                            const bool acc = dE < thr;
-                            if (acc) { sx[si] = px; sy[si] = py; sz[si] = pz; }
-                            nacc += acc ? 1u : 0u;
-                            nrej += acc ? 0u : 1u;
+                    for (int m = 0; m < NPL; m++) {
+                        const unsigned a8 = n0.ab[m] & 0xFFFF, b8 = n0.ab[m] >> 16;
+                        if (MIXED) {
+                            const char *pxy = (const char *)sx, *pzl = (const char *)sz;
+                            const double2 pa = *(const double2 *)(pxy + 2 * a8), pb = *(const double2 *)(pxy + 2 * b8);
+                            const double2 za = *(const double2 *)(pzl + 2 * a8), zb = *(const double2 *)(pzl + 2 * b8);
+                            ax[m] = pa.x; ay[m] = pa.y; az[m] = za.x; la[m] = za.y;
+                            bx[m] = pb.x; by[m] = pb.y; bz[m] = zb.x; lb[m] = zb.y;
+                        } else {
+                            ax[m] = *(const double *)((const char *)sx + a8);
+                            ay[m] = *(const double *)((const char *)sy + a8);
+                            az[m] = *(const double *)((const char *)sz + a8);
+                            bx[m] = *(const double *)((const char *)sx + b8);
+                            by[m] = *(const double *)((const char *)sy + b8);
+                            bz[m] = *(const double *)((const char *)sz + b8);
                         }
                     }
-                    if constexpr (LOOKAHEAD) cur = prepare(pk_next, bn + group - p0);
-                    if (last) __syncthreads();   // the colour is done before the next one reads it
+                    const double pv = prop[4 * pq + comp], ov = own[ZS * si];
+#pragma unroll
+                    for (int m = 0; m < NPL; m++) {
+                        double mx, my, mz;
+                        if (MIXED) {
+                            mx = la[m] * ax[m] + lb[m] * bx[m];
+                            my = la[m] * ay[m] + lb[m] * by[m];
+                            mz = la[m] * az[m] + lb[m] * bz[m];
+                            if (m == 0) {
+                                gx_ = nnf * (ax[0] + bx[0]); gy_ = nnf * (ay[0] + by[0]); gz_ = nnf * (az[0] + bz[0]);
+                            }
+                        } else {
+                            mx = ax[m] + bx[m]; my = ay[m] + by[m]; mz = az[m] + bz[m];
+                        }
+                        const double f = w3[m] * (nx[m] * mx + ny[m] * my + nz[m] * mz);
+                        hx_ = fma(f, nx[m], m == 0 ? (MIXED ? w[m] * mx : fma(w[m], mx, E0)) : fma(w[m], mx, hx_));
+                        hy_ = fma(f, ny[m], m == 0 ? (MIXED ? w[m] * my : fma(w[m], my, E1)) : fma(w[m], my, hy_));
+                        hz_ = fma(f, nz[m], m == 0 ? (MIXED ? w[m] * mz : fma(w[m], mz, E2)) : fma(w[m], mz, hz_));
+                    }
+                    double Li = 1.0;
+                    if (MIXED) {
+                        Li = lane_bcast<3, G>(ov);
+                        hx_ = fma(Li, hx_, fma(-J, gx_, E0)); hy_ = fma(Li, hy_, fma(-J, gy_, E1));
+                        hz_ = fma(Li, hz_, fma(-J, gz_, E2));
+                    }
+                    const double d = pv - ov;
+                    double dE = lane_bcast<0, G>(d) * hx_ + lane_bcast<1, G>(d) * hy_ + lane_bcast<2, G>(d) * hz_;
+                    if (K > 0.0) {
+                        asm volatile("" ::: "memory");
+                        dE -= Kp * (fabs(pv) - fabs(ov));
+                    }
+                    dE = group_sum_dpp<G>(dE);
+                    // (the fence keeps the exchange above the branch, where lane 3 is on)
+                    double thr = lane_bcast<3, G>(pv);
+                    asm volatile("" : "+v"(thr), "+v"(Li));
+                    if (writer && Li != 0.0) {
+                        nvis++;
+                        if (dE < thr) {
+                            own[ZS * si] = pv;
+                            nacc++;
+                        }
+                    }
                 }
+                if (__builtin_amdgcn_readfirstlane(e0) & kStepBarrier) __syncthreads();
+                e0 = e1; n0 = n1;
+                e1 = e2; n1 = n2;
             }
-            k0 = k1;
         }
     }
 
-    // ---- write back and count ----
+    // ---- count, write back ----
+    if (part == 0 && nvis) {
+        if (nacc) atomicAdd(&s_cnt[0], nacc);
+        atomicAdd(&s_cnt[1], nvis - nacc);
+    }
+    __syncthreads();
+    if (tid < 2) atomicAdd(t.counters + 2 * r + tid, (unsigned long long)s_cnt[tid]);
     for (int i = tid; i < N; i += BLK) {
         double4 v;
-        v.x = sx[i]; v.y = sy[i]; v.z = sz[i];
-        v.w = MIXED ? sl[i] : rep.L0;
+        v.x = sx[ZS * i]; v.y = sy[ZS * i]; v.z = sz[ZS * i];
+        v.w = MIXED ? sz[2 * i + 1] : rep.L0;
         lat[i] = v;
-    }
-    unsigned long long ca = nacc, cr = nrej;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-        ca += __shfl_xor(ca, o, 64);
-        cr += __shfl_xor(cr, o, 64);
-    }
-    __shared__ unsigned long long s_cnt[2 * (BLK / 64)];
-    if ((tid & 63) == 0) { s_cnt[2 * (tid >> 6)] = ca; s_cnt[2 * (tid >> 6) + 1] = cr; }
-    __syncthreads();
-    if (tid == 0) {
-        unsigned long long A_ = 0, R_ = 0;
-        for (int w_ = 0; w_ < BLK / 64; w_++) { A_ += s_cnt[2 * w_]; R_ += s_cnt[2 * w_ + 1]; }
-        t.counters[2 * r] += A_;
-        t.counters[2 * r + 1] += R_;
     }
 }
 
