@@ -96,10 +96,12 @@ struct sn_ctx {
     std::vector<std::vector<int32_t>> torus_order, torus_cstart;   // per replica: sites by colour, colour starts
     int torus_ncol = 0;                                             // colours per sweep (shorter colourings padded)
     int torus_G = 0, torus_NPL = 0, torus_blk = 0, torus_ms = 0, torus_mc = 0, torus_pc = 0;
-    int *d_torus_box_of = nullptr, *d_torus_sites = nullptr, *d_torus_entries = nullptr, *d_torus_chunks = nullptr;
+    int *d_torus_box_of = nullptr, *d_torus_sites = nullptr, *d_torus_chunks = nullptr;
     TorusBox *d_torus_boxes = nullptr;
-    unsigned short *d_torus_near = nullptr;
+    int2 *d_torus_own[2] = {nullptr, nullptr};   // round tables for uniform and mixed lengths
+    int *d_torus_near[2] = {nullptr, nullptr};
     int torus_max_chunks = 0;
+    bool torus_two = false;   // two sites per group and round
     unsigned long long *d_rep_counters = nullptr;   // 2 per replica (torus sweeps)
     bool can_sweep = false;
     std::string sweep_err;
@@ -345,10 +347,16 @@ const char *sn_last_error(const sn_ctx *ctx) { return ctx ? ctx->err.c_str() : "
 // when a replica is too large for LDS or no such colouring exists.
 constexpr int kTorusMaxIndex = 128;
 
+static int torus_site_bytes(const sn_ctx *c, bool mixed)
+{
+    const int bytes = torus_address((c->torus_ms + 255) & ~255, mixed);   // whole blocks
+    return (bytes + 15) & ~15;
+}
+
 static size_t torus_lds(const sn_ctx *c, bool mixed)
 {
-    return (size_t)((((mixed ? 4 : 3) * c->torus_ms + 1) & ~1) + 4 * c->torus_pc) * sizeof(double) +
-           (size_t)2 * (c->torus_max_chunks + 1) * sizeof(int);
+    return (size_t)torus_site_bytes(c, mixed) + (size_t)4 * c->torus_pc * sizeof(double) +
+           (size_t)(2 * (c->torus_max_chunks + 1) + 2) * sizeof(int) + (size_t)c->torus_ms * sizeof(unsigned short);
 }
 
 // lanes per site, pairs per lane and threads for npairs pairs and colours of
@@ -461,10 +469,14 @@ static int setup_torus(sn_ctx *c)
     // tables of each box size: the sites by colour, the rounds' entries and
     // neighbours, the runs of colours whose proposals are drawn together
     const int NG = blk / G;
+    // two sites per group and round where a colour has more sites than the
+    // workgroup has groups (and an instance holds them)
+    c->torus_two = c->torus_mc > NG && pick_torus(G, NPL, false, blk, true);
+    const int R = c->torus_two ? 2 : 1;
     const std::vector<Offset> pairs = neighbour_pairs(c->rc, c->two_d);
     std::vector<TorusBox> boxes;
-    std::vector<int> box_of, sites, entries, chunks;
-    std::vector<unsigned short> near;
+    std::vector<int> box_of, sites, chunks, near[2];
+    std::vector<int2> own[2];
     std::map<std::array<int, 3>, int> known;
     for (int r = 0; r < c->R; r++) {
         const ReplicaGeom &g = c->geom[r];
@@ -474,9 +486,8 @@ static int setup_torus(sn_ctx *c)
         const std::vector<int32_t> &o = c->torus_order[r], &cst = c->torus_cstart[r];
         TorusBox b{};
         b.sites_off = (int)sites.size();
-        b.entry_off = (int)entries.size();
         b.chunk_off = (int)chunks.size();
-        b.near_off = (long long)near.size();
+        b.round_off = (long long)own[0].size();
         sites.insert(sites.end(), o.begin(), o.end());
         const int ncol = (int)cst.size() - 1;
         int p0 = 0;   // first site of the run of colours
@@ -487,24 +498,33 @@ static int setup_torus(sn_ctx *c)
                 chunks.push_back(p0);
                 b.nchunks++;
             }
-            for (int b0 = cst[k]; b0 < cst[k + 1]; b0 += NG, b.nrounds++) {
-                const bool last = b0 + NG >= cst[k + 1];
-                for (int q = 0; q < NG; q++) {
+            for (int b0 = cst[k]; b0 < cst[k + 1]; b0 += R * NG, b.nrounds++) {
+                const bool last = b0 + R * NG >= cst[k + 1];
+                for (int q = 0; q < R * NG; q++) {
                     const bool idle = b0 + q >= cst[k + 1];
-                    const int si = idle ? o[0] : o[b0 + q];
-                    entries.push_back(torus_entry(si, idle ? 0 : b0 + q - p0, last, idle));
+                    const int si = idle ? o[0] : o[b0 + q], slot = idle ? 0 : b0 + q - p0;
                     const int z = si % g.Z, y = si / g.Z % g.Y, x = si / (g.Z * g.Y);
-                    auto at8 = [&](int a, int bb, int cc) {
-                        a = (a + g.X) % g.X; bb = (bb + g.Y) % g.Y; cc = (cc + g.Z) % g.Z;
-                        return (unsigned short)(8 * ((a * g.Y + bb) * g.Z + cc));
+                    auto wrapped = [&](int a, int bb, int cc) {   // (|offset| < axis)
+                        a += a < 0 ? g.X : a >= g.X ? -g.X : 0;
+                        bb += bb < 0 ? g.Y : bb >= g.Y ? -g.Y : 0;
+                        cc += cc < 0 ? g.Z : cc >= g.Z ? -g.Z : 0;
+                        return (a * g.Y + bb) * g.Z + cc;
                     };
-                    for (int part = 0; part < G; part++)
+                    for (int part = 0; part < G; part++) {
+                        for (int mixed = 0; mixed < 2; mixed++)
+                            own[mixed].push_back(int2{(torus_address(si, mixed) + torus_component(part & 3, mixed)) |
+                                                          (last ? kLast : 0) | (idle ? kIdle : 0),
+                                                      torus_site_bytes(c, mixed) + 32 * slot + 8 * (part & 3)});
                         for (int m = 0; m < NPL; m++) {
                             Offset d{0, 0, 0, 0};   // a padded pair: the site itself, with no weight
                             if (part + m * G < np) d = pairs[part + m * G];
-                            near.push_back(at8(x + d.dx, y + d.dy, z + d.dz));
-                            near.push_back(at8(x - d.dx, y - d.dy, z - d.dz));
+                            const int sa = wrapped(x + d.dx, y + d.dy, z + d.dz), sb = wrapped(x - d.dx, y - d.dy, z - d.dz);
+                            for (int mixed = 0; mixed < 2; mixed++) {
+                                near[mixed].push_back(torus_address(sa, mixed));
+                                near[mixed].push_back(torus_address(sb, mixed));
+                            }
                         }
+                    }
                 }
             }
         }
@@ -514,21 +534,22 @@ static int setup_torus(sn_ctx *c)
         boxes.push_back(b);
     }
     // (four arrays, proposals and an int per site: what a replica may take)
-    if ((size_t)4 * (c->torus_ms + c->torus_pc) * sizeof(double) + (size_t)c->torus_ms * sizeof(int) > 150 * 1024 ||
-        c->torus_ms > kTorusMaxSites)
+    if ((size_t)4 * (c->torus_ms + c->torus_pc) * sizeof(double) + (size_t)c->torus_ms * sizeof(int) > 150 * 1024)
         return fail(c, SN_ERR_UNSUPPORTED, "whole-lattice sweep: a replica does not fit in LDS (" +
                                                std::to_string(c->torus_ms) + " sites)");
     int st;
     for (int m = 0; m < 2; m++) {
-        const void *f = (const void *)pick_torus(G, NPL, m == 1, blk);
+        const void *f = (const void *)pick_torus(G, NPL, m == 1, blk, c->torus_two);
         if (!f) return fail(c, SN_ERR_UNSUPPORTED, "whole-lattice sweep: no kernel for this cutoff");
         HIPCHK(c, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)torus_lds(c, true)));
     }
     if ((st = upload(c, &c->d_torus_box_of, box_of))) return st;
     if ((st = upload(c, &c->d_torus_boxes, boxes))) return st;
     if ((st = upload(c, &c->d_torus_sites, sites))) return st;
-    if ((st = upload(c, &c->d_torus_entries, entries))) return st;
-    if ((st = upload(c, &c->d_torus_near, near))) return st;
+    for (int m = 0; m < 2; m++) {
+        if ((st = upload(c, &c->d_torus_own[m], own[m]))) return st;
+        if ((st = upload(c, &c->d_torus_near[m], near[m]))) return st;
+    }
     if ((st = upload(c, &c->d_torus_chunks, chunks))) return st;
     std::vector<unsigned long long> z(2 * c->R, 0ull);
     if ((st = upload(c, &c->d_rep_counters, z))) return st;
@@ -902,7 +923,8 @@ int sn_destroy(sn_ctx *c)
                     c->d_offs, c->d_sweep,
                     c->d_counters, c->d_partials, c->d_result, c->d_radial, c->d_radial_bins,
                     c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
-                    c->d_torus_sites, c->d_torus_entries, c->d_torus_near, c->d_torus_chunks, c->d_rep_counters, c->d_stage};
+                    c->d_torus_sites, c->d_torus_own[0], c->d_torus_own[1], c->d_torus_near[0],
+                    c->d_torus_near[1], c->d_torus_chunks, c->d_rep_counters, c->d_stage};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_result) (void)hipHostFree(c->h_result);
@@ -1147,13 +1169,13 @@ static int launch_torus(sn_ctx *c, int nsw, std::vector<hipEvent_t> *events)
     TorusArgs t;
     t.lat = c->d_lat; t.reps = c->d_reps; t.pairs = c->d_pairs;
     t.box_of = c->d_torus_box_of; t.boxes = c->d_torus_boxes; t.sites = c->d_torus_sites;
-    t.entries = c->d_torus_entries; t.nears = c->d_torus_near; t.chunks = c->d_torus_chunks;
+    t.owns = c->d_torus_own[mixed]; t.nears = c->d_torus_near[mixed]; t.chunks = c->d_torus_chunks;
     t.sweep_ctr = c->d_sweep; t.counters = c->d_rep_counters;
-    t.max_sites = c->torus_ms; t.prop_cap = c->torus_pc;
+    t.site_bytes = torus_site_bytes(c, mixed); t.prop_cap = c->torus_pc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (events && (event_pair(c, events, &e0, &e1) || hipEventRecord(e0, c->stream) != hipSuccess))
         return fail(c, SN_ERR_HIP, "timing events");
-    hipLaunchKernelGGL(pick_torus(c->torus_G, c->torus_NPL, mixed, c->torus_blk), dim3(c->R), dim3(c->torus_blk),
+    hipLaunchKernelGGL(pick_torus(c->torus_G, c->torus_NPL, mixed, c->torus_blk, c->torus_two), dim3(c->R), dim3(c->torus_blk),
                        torus_lds(c, mixed), c->stream, t, nsw);
     HIPCHK(c, hipGetLastError());
     if (events) HIPCHK(c, hipEventRecord(e1, c->stream));

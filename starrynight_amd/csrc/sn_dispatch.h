@@ -23,8 +23,9 @@ constexpr int kFixedRegion = 14 * 14 * 14;
 // chunks of kBlock selects the compile-time-stride instance where one is built
 SweepFn pick_sweep(int G, int NPL, bool mixed, int blk, int max_region = 0, int prop_chunk = 0);
 typedef void (*TorusFn)(TorusArgs, int);
-// whole-lattice sweep kernel of small replicas (or null)
-TorusFn pick_torus(int G, int NPL, bool mixed, int blk);
+// whole-lattice sweep kernel of small replicas (or null); two: two sites per
+// group and round (at most 512 threads: 1024 leave 128 registers a lane)
+TorusFn pick_torus(int G, int NPL, bool mixed, int blk, bool two = false);
 // field-update kernel for DipoleCutOff rc (1..5) or null
 FieldFn pick_field(int rc, bool two_d, bool mixed);
 FieldFn pick_field_rc1(bool two_d, bool mixed);

@@ -30,11 +30,19 @@ SweepFn pick_sweep(int G, int NPL, bool mixed, int blk, int max_region, int prop
     return nullptr;
 }
 
-TorusFn pick_torus(int G, int NPL, bool mixed, int blk)
+template <int G, int NPL, int BLK>
+static TorusFn torus_instance(bool mixed, bool two)
 {
-#define SN_CASE(g, n, b)                                                                          \
-    if (G == g && NPL == n && blk == b) return mixed ? (TorusFn)torus_sweep_kernel<g, n, true, b>   \
-                                                     : (TorusFn)torus_sweep_kernel<g, n, false, b>;
+    if constexpr (BLK <= 512)
+        if (two) return mixed ? (TorusFn)torus_sweep_kernel<G, NPL, true, BLK, 2>
+                              : (TorusFn)torus_sweep_kernel<G, NPL, false, BLK, 2>;
+    return two ? nullptr : mixed ? (TorusFn)torus_sweep_kernel<G, NPL, true, BLK, 1>
+                                 : (TorusFn)torus_sweep_kernel<G, NPL, false, BLK, 1>;
+}
+
+TorusFn pick_torus(int G, int NPL, bool mixed, int blk, bool two)
+{
+#define SN_CASE(g, n, b) if (G == g && NPL == n && blk == b) return torus_instance<g, n, b>(mixed, two);
     SN_CASE(4, 4, 256) SN_CASE(8, 4, 256) SN_CASE(16, 4, 256) SN_CASE(32, 2, 1024) SN_CASE(64, 2, 1024)
     SN_CASE(8, 2, 256) SN_CASE(16, 1, 256) SN_CASE(16, 1, 512) SN_CASE(16, 2, 512) SN_CASE(32, 1, 512)
     SN_CASE(16, 1, 1024) SN_CASE(8, 2, 512)

@@ -22,10 +22,9 @@ namespace sn {
 // One box size: where its tables start.
 struct TorusBox {
     int sites_off;             // sites by colour (linear index), N of them
-    int entry_off, nrounds;    // NG step_entry's per round; rounds of one sweep
+    int nrounds;               // of one sweep
     int chunk_off, nchunks;    // first round and first site of each run of proposals (nchunks + 1 of both)
-    int pad;
-    long long near_off;        // 2 NPL shorts per lane and round
+    long long round_off;       // first of its lane records: R per lane and round
 };
 
 struct TorusArgs {
@@ -35,25 +34,59 @@ struct TorusArgs {
     const int *box_of;         // R entries
     const TorusBox *boxes;
     const int *sites;          // per box (sites_off)
-    const int *entries;        // per box (entry_off): site | slot << 13 by group, flags as step_entry
-    const unsigned short *nears;   // per box (near_off): 8 x site index of the lane's neighbours, + and - of each pair
+    // per box (round_off), round, site and lane, for the layout of the launch
+    // (uniform or mixed lengths):
+    const int2 *owns;          // LDS bytes of the lane's own component (with kLast, kIdle) and of its proposal's
+    const int *nears;          // 2 NPL: LDS bytes of its neighbours, + and - of each pair
     const int *chunks;         // per box (chunk_off)
     const unsigned *sweep_ctr;
     unsigned long long *counters;  // 2 per replica: accepted, rejected (accumulated)
-    int max_sites;             // stride of the staged arrays
+    int site_bytes;            // LDS bytes of the largest replica's sites
     int prop_cap;              // proposal slots (>= the largest colour): colours are drawn in
                                // runs of at most this many sites
 };
 
-// Entry of a lane group: site and proposal slot have 13 bits each (a replica
-// of at most kTorusMaxSites fits in LDS).
-constexpr int kTorusMaxSites = 8191;
-__host__ __device__ inline int torus_entry(int site, int slot, bool last, bool idle)
+// Flags in the low bits of an own component's LDS address: a colour's last
+// round (it ends with the barrier), a group without a site.
+constexpr int kLast = 1, kIdle = 2;
+
+// LDS layout in blocks of 256 sites, so that a site's components lie at fixed
+// distances from its address, which the reads take as immediate offsets (x, y
+// and z arrays a runtime stride apart cost two adds per neighbour): x, y and z
+// arrays of the block, or with mixed lengths (x, y) and (z, L) pairs.  The
+// distances are odd multiples of 8 or 16 bytes, so that a site's components
+// lie in different banks, and beyond the reach of a two-address read: blocks
+// of 64 with 512 bytes between x and y, which the compiler reads as one
+// read2st64 from one bank, ran 25 x 25 16% slower than the runtime strides.
+__host__ __device__ inline int torus_address(int site, bool mixed)
 {
-    return site | (slot << 13) | (last ? kStepBarrier : 0) | (idle ? kStepIdle : 0);
+    return (site >> 8) * (mixed ? 2 * 4112 : 3 * 2056) + (site & 255) * (mixed ? 16 : 8);
+}
+// of component c (x, y, z, L) relative to the site's address
+__host__ __device__ inline int torus_component(int c, bool mixed)
+{
+    return mixed ? (c >> 1) * 4112 + (c & 1) * 8 : (c < 3 ? c : 2) * 2056;
 }
 
-template <int G, int NPL, bool MIXED, int BLK>
+// LDS at a byte address: the kernel has no static LDS, so its dynamic array,
+// and with it torus_address, begins at 0.  (Through a pointer into the array
+// every read of a table's address cost an add of that zero.)
+typedef double lds_double2 __attribute__((ext_vector_type(2)));
+template <typename T>
+__device__ __forceinline__ T lds_load(int address)
+{
+    return *(const __attribute__((address_space(3))) T *)(uintptr_t)(unsigned)address;
+}
+__device__ __forceinline__ void lds_store(int address, double v)
+{
+    *(__attribute__((address_space(3))) double *)(uintptr_t)(unsigned)address = v;
+}
+
+// R sites per group and round, of one colour: with one (colours that fit the
+// groups) a round's latencies follow one another; two sites' reads, sums and
+// reductions overlap (64 x 12^3 at DipoleCutOff 3, 54 sites a colour on 16
+// groups, 10 sweeps: 710 -> 641 us).
+template <int G, int NPL, bool MIXED, int BLK, int R>
 __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nsweeps)
 {
     static_assert(G * NPL <= kPairSlots, "the pair table covers every lane's slots");
@@ -62,31 +95,30 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
     const RepDev rep = t.reps[r];
     const TorusBox box = t.boxes[t.box_of[r]];
     const int N = rep.X * rep.Y * rep.Z;
-    const int MS = t.max_sites, PS = t.prop_cap;
-    // as the tile sweep: x, y and z arrays, or (x, y) and (z, L) pairs
-    constexpr int ZS = MIXED ? 2 : 1;
-    double *sx = smem;
-    double *sy = MIXED ? sx + 1 : sx + MS;
-    double *sz = sx + 2 * MS;
-    double *prop = sx + (((MIXED ? 4 : 3) * MS + 1) & ~1);   // px, py, pz and threshold of slot k at prop[4 k]
-    int *s_chunk = (int *)(prop + 4 * PS);
+    constexpr int YO = MIXED ? 8 : 2056, ZO = 4112;   // torus_component of y and z
+    char *sites = (char *)smem;                               // torus_address, torus_component
+    double *prop = (double *)(sites + t.site_bytes);          // px, py, pz and threshold of slot k at prop[4 k]
+    int *s_chunk = (int *)(prop + 4 * t.prop_cap);
+    unsigned *s_cnt = (unsigned *)(s_chunk + 2 * (box.nchunks + 1));   // (no static LDS: sites begin at address 0)
+    unsigned short *s_site = (unsigned short *)(s_cnt + 2);   // sites by colour
     double4 *lat = t.lat + rep.base;
 
     // ---- the whole replica into LDS ----
     for (int i = tid; i < N; i += BLK) {
         const double4 v = lat[i];
+        char *p = sites + torus_address(i, MIXED);
         if (MIXED) {
-            ((double2 *)sx)[i] = make_double2(v.x, v.y);
-            ((double2 *)sz)[i] = make_double2(v.z, v.w);
+            *(double2 *)p = make_double2(v.x, v.y);
+            *(double2 *)(p + ZO) = make_double2(v.z, v.w);
         } else {
-            sx[i] = v.x; sy[i] = v.y; sz[i] = v.z;
+            *(double *)p = v.x; *(double *)(p + YO) = v.y; *(double *)(p + ZO) = v.z;
         }
+        s_site[i] = (unsigned short)t.sites[box.sites_off + i];
     }
     for (int i = tid; i < 2 * (box.nchunks + 1); i += BLK) s_chunk[i] = t.chunks[box.chunk_off + i];
 
     // ---- this lane's share of the +-r pairs ----
-    const int part = tid % G, group = tid / G;
-    constexpr int NG = BLK / G;
+    const int part = tid % G;
     double nx[NPL], ny[NPL], nz[NPL], w[NPL], w3[NPL], nnf = 0.0;
 #pragma unroll
     for (int m = 0; m < NPL; m++) {
@@ -106,127 +138,176 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
         for (int m = 0; m < NPL; m++) { w[m] *= LL; w3[m] *= LL; }
         w[0] -= nnf * J;
     }
-    const int comp = part & 3;
-    double *own = MIXED ? sx + (comp >> 1) * 2 * MS + (comp & 1) : sx + (comp < 3 ? comp : 2) * MS;
     const double Kp = part < 2 ? K : 0.0;
     const bool writer = part < 3 && (MIXED || rep.L0 != 0.0);   // vacancies never move and are not counted
     unsigned nacc = 0, nvis = 0;   // accepted (on a group's first lane), visited
-    __shared__ unsigned s_cnt[2];
     if (tid < 2) s_cnt[tid] = 0;
 
-    // ---- the round tables, two rounds ahead of their use ----
+    // ---- the round tables, three rounds ahead (a load issued one round ahead
+    // is still on its way from L2 when the round begins) ----
     struct Near {
-        unsigned ab[NPL];   // 8 x site of the pair's + neighbour, - neighbour << 16
+        int a[2 * NPL];   // + and - neighbour of each pair
     };
-    const int *entries = t.entries + box.entry_off + group;
-    const Near *nears = (const Near *)(t.nears + box.near_off) + tid;
-    int e0, e1, e2;
-    Near n0, n1, n2;
+    struct Round {
+        int2 own[R];
+        Near n[R];
+    };
+    const int2 *owns = t.owns + box.round_off + tid;
+    const Near *nears = (const Near *)t.nears + box.round_off + tid;
+    Round q0, q1, q2;
     int ahead = 0;   // the round loaded next (the sweep's rounds repeat)
-    auto fetch = [&](int &e, Near &n) __attribute__((always_inline)) {
-        e = entries[ahead * NG];
-        n = nears[(long long)ahead * BLK];
+    auto fetch = [&](Round &q) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < R; i++) {
+            q.own[i] = owns[(long long)(ahead * R + i) * BLK];
+            q.n[i] = nears[(long long)(ahead * R + i) * BLK];
+        }
         ahead = ahead + 1 < box.nrounds ? ahead + 1 : 0;
     };
-    fetch(e0, n0);
-    fetch(e1, n1);
+    fetch(q0);
+    fetch(q1);
+    fetch(q2);
+    const unsigned sweep0 = t.sweep_ctr[r];
     __syncthreads();
 
     for (int s = 0; s < nsweeps; s++) {
-        const unsigned sweep = t.sweep_ctr[r] + (unsigned)s;
+        const unsigned sweep = sweep0 + (unsigned)s;
         for (int ch = 0; ch < box.nchunks; ch++) {
-            // ---- proposals of a run of colours, two sites per lane at a time ----
+            // ---- proposals of a run of colours, two sites per lane at a time
+            // (one where no lane of the wave has a second) ----
             const int p0 = s_chunk[2 * ch + 1], np = s_chunk[2 * ch + 3] - p0;
+            auto store = [&](int k, double px, double py, double pz, double u) __attribute__((always_inline)) {
+                ((double2 *)prop)[2 * k] = make_double2(px, py);
+                ((double2 *)prop)[2 * k + 1] = make_double2(pz, metropolis_threshold(u, rep.beta, rbeta));
+            };
             for (int i = tid; i < np; i += 2 * BLK) {
                 const bool two = i + BLK < np;
-                const uint32_t site[2] = {(uint32_t)t.sites[box.sites_off + p0 + i],
-                                          (uint32_t)t.sites[box.sites_off + p0 + (two ? i + BLK : i)]};
-                double px[2], py[2], pz[2], u[2];
-                counter_draws<2>(rep.seed, (uint32_t)r, sweep, site, rep.constrain_to_x, px, py, pz, u);
-#pragma unroll
-                for (int q = 0; q < 2; q++)
-                    if (q == 0 || two) {
-                        ((double2 *)prop)[2 * (i + q * BLK)] = make_double2(px[q], py[q]);
-                        ((double2 *)prop)[2 * (i + q * BLK) + 1] =
-                            make_double2(pz[q], metropolis_threshold(u[q], rep.beta, rbeta));
-                    }
+                if (__any(two)) {
+                    const uint32_t site[2] = {s_site[p0 + i], s_site[p0 + (two ? i + BLK : i)]};
+                    double px[2], py[2], pz[2], u[2];
+                    counter_draws<2>(rep.seed, (uint32_t)r, sweep, site, rep.constrain_to_x, px, py, pz, u);
+                    store(i, px[0], py[0], pz[0], u[0]);
+                    if (two) store(i + BLK, px[1], py[1], pz[1], u[1]);
+                } else {
+                    double px, py, pz, u;
+                    counter_draw(rep.seed, (uint32_t)r, sweep, s_site[p0 + i], rep.constrain_to_x, px, py, pz, u);
+                    store(i, px, py, pz, u);
+                }
             }
             const int r0 = __builtin_amdgcn_readfirstlane(s_chunk[2 * ch]);
             const int r1 = __builtin_amdgcn_readfirstlane(s_chunk[2 * ch + 2]);
             __syncthreads();
-            // ---- the run's rounds: every group decides one site; a colour's
+            // ---- the run's rounds: every group decides its sites; a colour's
             // last round ends with the barrier (before it, rounds of a colour
             // are independent of each other) ----
-            for (int rd = r0; rd < r1; rd++) {
-                fetch(e2, n2);
-                if (e0 >= 0) {   // whole groups are active or not
-                    const int si = e0 & 8191, pq = (e0 >> 13) & 8191;
-                    double hx_, hy_, hz_, gx_, gy_, gz_;
-                    double ax[NPL], ay[NPL], az[NPL], bx[NPL], by[NPL], bz[NPL], la[NPL], lb[NPL];
-#pragma unroll
-                    for (int m = 0; m < NPL; m++) {
-                        const unsigned a8 = n0.ab[m] & 0xFFFF, b8 = n0.ab[m] >> 16;
+            auto round = [&](const Round &q) __attribute__((always_inline)) {
+                // one site: groups without one (whole DPP rows or quads) skip
+                // the round.  Two: waves without any do; a group without one
+                // runs on the site its entry names and drops the result, so
+                // that both sites' instructions are one stream.
+                if (R == 1 ? !(q.own[0].x & kIdle) : __any(!(q.own[0].x & kIdle))) {
+                    double ax[R][NPL], ay[R][NPL], az[R][NPL], bx[R][NPL], by[R][NPL], bz[R][NPL], la[R][NPL], lb[R][NPL];
+                    double pv[R], ov[R], dE[R], thr[R], Li[R];
+                    auto pair_reads = [&](int i, int m) __attribute__((always_inline)) {
+                        const int pa = q.n[i].a[2 * m], pb = q.n[i].a[2 * m + 1];
                         if (MIXED) {
-                            const char *pxy = (const char *)sx, *pzl = (const char *)sz;
-                            const double2 pa = *(const double2 *)(pxy + 2 * a8), pb = *(const double2 *)(pxy + 2 * b8);
-                            const double2 za = *(const double2 *)(pzl + 2 * a8), zb = *(const double2 *)(pzl + 2 * b8);
-                            ax[m] = pa.x; ay[m] = pa.y; az[m] = za.x; la[m] = za.y;
-                            bx[m] = pb.x; by[m] = pb.y; bz[m] = zb.x; lb[m] = zb.y;
+                            const lds_double2 xya = lds_load<lds_double2>(pa), zla = lds_load<lds_double2>(pa + ZO);
+                            const lds_double2 xyb = lds_load<lds_double2>(pb), zlb = lds_load<lds_double2>(pb + ZO);
+                            ax[i][m] = xya.x; ay[i][m] = xya.y; az[i][m] = zla.x; la[i][m] = zla.y;
+                            bx[i][m] = xyb.x; by[i][m] = xyb.y; bz[i][m] = zlb.x; lb[i][m] = zlb.y;
                         } else {
-                            ax[m] = *(const double *)((const char *)sx + a8);
-                            ay[m] = *(const double *)((const char *)sy + a8);
-                            az[m] = *(const double *)((const char *)sz + a8);
-                            bx[m] = *(const double *)((const char *)sx + b8);
-                            by[m] = *(const double *)((const char *)sy + b8);
-                            bz[m] = *(const double *)((const char *)sz + b8);
+                            ax[i][m] = lds_load<double>(pa);
+                            ay[i][m] = lds_load<double>(pa + YO);
+                            az[i][m] = lds_load<double>(pa + ZO);
+                            bx[i][m] = lds_load<double>(pb);
+                            by[i][m] = lds_load<double>(pb + YO);
+                            bz[i][m] = lds_load<double>(pb + ZO);
                         }
-                    }
-                    const double pv = prop[4 * pq + comp], ov = own[ZS * si];
+                        if (m + 1 == NPL) {
+                            pv[i] = lds_load<double>(q.own[i].y);
+                            ov[i] = lds_load<double>(q.own[i].x & ~7);
+                        }
+                    };
+                    // two sites: reads run two pairs ahead of the sums (see the
+                    // tile sweep; 64 x 12^3, 10 sweeps: 641 us, all reads
+                    // first 702)
+                    constexpr int AHEAD = R == 1 || R * NPL < 2 ? R * NPL : 2;
 #pragma unroll
-                    for (int m = 0; m < NPL; m++) {
-                        double mx, my, mz;
-                        if (MIXED) {
-                            mx = la[m] * ax[m] + lb[m] * bx[m];
-                            my = la[m] * ay[m] + lb[m] * by[m];
-                            mz = la[m] * az[m] + lb[m] * bz[m];
-                            if (m == 0) {
-                                gx_ = nnf * (ax[0] + bx[0]); gy_ = nnf * (ay[0] + by[0]); gz_ = nnf * (az[0] + bz[0]);
+                    for (int k = 0; k < AHEAD; k++) pair_reads(k / NPL, k % NPL);
+#pragma unroll
+                    for (int i = 0; i < R; i++) {
+                        double hx_, hy_, hz_, gx_, gy_, gz_;
+#pragma unroll
+                        for (int m = 0; m < NPL; m++) {
+                            if (R > 1) asm volatile("" ::: "memory");
+                            double mx, my, mz;
+                            if (MIXED) {
+                                mx = la[i][m] * ax[i][m] + lb[i][m] * bx[i][m];
+                                my = la[i][m] * ay[i][m] + lb[i][m] * by[i][m];
+                                mz = la[i][m] * az[i][m] + lb[i][m] * bz[i][m];
+                                if (m == 0) {
+                                    gx_ = nnf * (ax[i][0] + bx[i][0]); gy_ = nnf * (ay[i][0] + by[i][0]);
+                                    gz_ = nnf * (az[i][0] + bz[i][0]);
+                                }
+                            } else {
+                                mx = ax[i][m] + bx[i][m]; my = ay[i][m] + by[i][m]; mz = az[i][m] + bz[i][m];
                             }
-                        } else {
-                            mx = ax[m] + bx[m]; my = ay[m] + by[m]; mz = az[m] + bz[m];
+                            const double f = w3[m] * (nx[m] * mx + ny[m] * my + nz[m] * mz);
+                            hx_ = fma(f, nx[m], m == 0 ? (MIXED ? w[m] * mx : fma(w[m], mx, E0)) : fma(w[m], mx, hx_));
+                            hy_ = fma(f, ny[m], m == 0 ? (MIXED ? w[m] * my : fma(w[m], my, E1)) : fma(w[m], my, hy_));
+                            hz_ = fma(f, nz[m], m == 0 ? (MIXED ? w[m] * mz : fma(w[m], mz, E2)) : fma(w[m], mz, hz_));
+                            if (R > 1) asm volatile("" : "+v"(hx_), "+v"(hy_), "+v"(hz_) : : "memory");
+                            const int next = i * NPL + m + AHEAD;
+                            if (next < R * NPL) pair_reads(next / NPL, next % NPL);
                         }
-                        const double f = w3[m] * (nx[m] * mx + ny[m] * my + nz[m] * mz);
-                        hx_ = fma(f, nx[m], m == 0 ? (MIXED ? w[m] * mx : fma(w[m], mx, E0)) : fma(w[m], mx, hx_));
-                        hy_ = fma(f, ny[m], m == 0 ? (MIXED ? w[m] * my : fma(w[m], my, E1)) : fma(w[m], my, hy_));
-                        hz_ = fma(f, nz[m], m == 0 ? (MIXED ? w[m] * mz : fma(w[m], mz, E2)) : fma(w[m], mz, hz_));
-                    }
-                    double Li = 1.0;
-                    if (MIXED) {
-                        Li = lane_bcast<3, G>(ov);
-                        hx_ = fma(Li, hx_, fma(-J, gx_, E0)); hy_ = fma(Li, hy_, fma(-J, gy_, E1));
-                        hz_ = fma(Li, hz_, fma(-J, gz_, E2));
-                    }
-                    const double d = pv - ov;
-                    double dE = lane_bcast<0, G>(d) * hx_ + lane_bcast<1, G>(d) * hy_ + lane_bcast<2, G>(d) * hz_;
-                    if (K > 0.0) {
-                        asm volatile("" ::: "memory");
-                        dE -= Kp * (fabs(pv) - fabs(ov));
-                    }
-                    dE = group_sum_dpp<G>(dE);
-                    // (the fence keeps the exchange above the branch, where lane 3 is on)
-                    double thr = lane_bcast<3, G>(pv);
-                    asm volatile("" : "+v"(thr), "+v"(Li));
-                    if (writer && Li != 0.0) {
-                        nvis++;
-                        if (dE < thr) {
-                            own[ZS * si] = pv;
-                            nacc++;
+                        Li[i] = 1.0;
+                        if (MIXED) {
+                            Li[i] = lane_bcast<3, G>(ov[i]);
+                            hx_ = fma(Li[i], hx_, fma(-J, gx_, E0)); hy_ = fma(Li[i], hy_, fma(-J, gy_, E1));
+                            hz_ = fma(Li[i], hz_, fma(-J, gz_, E2));
                         }
+                        const double d = pv[i] - ov[i];
+                        dE[i] = lane_bcast<0, G>(d) * hx_ + lane_bcast<1, G>(d) * hy_ + lane_bcast<2, G>(d) * hz_;
+                        if (K > 0.0) {
+                            asm volatile("" ::: "memory");
+                            dE[i] -= Kp * (fabs(pv[i]) - fabs(ov[i]));
+                        }
+                        thr[i] = lane_bcast<3, G>(pv[i]);
                     }
+#pragma unroll
+                    for (int i = 0; i < R; i++) {
+                        dE[i] = group_sum_dpp<G>(dE[i]);
+                        // (the fence keeps the exchanges above the branch, where every lane is on)
+                        asm volatile("" : "+v"(dE[i]), "+v"(thr[i]), "+v"(Li[i]));
+                    }
+#pragma unroll
+                    for (int i = 0; i < R; i++)
+                        if (writer && (!MIXED || Li[i] != 0.0) && (R == 1 || !(q.own[i].x & kIdle))) {
+                            nvis++;
+                            if (dE[i] < thr[i]) {
+                                lds_store(q.own[i].x & ~7, pv[i]);
+                                nacc++;
+                            }
+                        }
                 }
-                if (__builtin_amdgcn_readfirstlane(e0) & kStepBarrier) __syncthreads();
-                e0 = e1; n0 = n1;
-                e1 = e2; n1 = n2;
+                if (__builtin_amdgcn_readfirstlane(q.own[0].x) & kLast) __syncthreads();
+            };
+            // (three copies of the round: rotating one register set into the
+            // next would wait for the loads just issued)
+            int rd = r0;
+            for (; rd + 3 <= r1; rd += 3) {
+                round(q0);
+                fetch(q0);
+                round(q1);
+                fetch(q1);
+                round(q2);
+                fetch(q2);
+            }
+            for (; rd < r1; rd++) {
+                round(q0);
+                q0 = q1;
+                q1 = q2;
+                fetch(q2);
             }
         }
     }
@@ -239,9 +320,12 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
     __syncthreads();
     if (tid < 2) atomicAdd(t.counters + 2 * r + tid, (unsigned long long)s_cnt[tid]);
     for (int i = tid; i < N; i += BLK) {
+        const char *p = sites + torus_address(i, MIXED);
         double4 v;
-        v.x = sx[ZS * i]; v.y = sy[ZS * i]; v.z = sz[ZS * i];
-        v.w = MIXED ? sz[2 * i + 1] : rep.L0;
+        v.x = *(const double *)p;
+        v.y = *(const double *)(p + YO);
+        v.z = *(const double *)(p + ZO);
+        v.w = MIXED ? *(const double *)(p + ZO + 8) : rep.L0;
         lat[i] = v;
     }
 }
