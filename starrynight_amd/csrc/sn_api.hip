@@ -13,6 +13,7 @@
 
 #include "../../include/starrynight_amd.h"
 #include "sn_aux_kernels.h"
+#include "sn_radial.h"
 #include "sn_dispatch.h"
 #include "sn_schedule.h"
 
@@ -65,13 +66,14 @@ struct sn_ctx {
     int max_steps = 0;   // longest step table of a tile shape (field kernel)
     int max_tile_padded = 0;   // largest padded tile (field kernel's tile-order arrays)
     PairDev *d_pairs = nullptr, *d_offs = nullptr;
-    RadialOff *d_radial = nullptr;   // radial-order offsets sorted by r^2 (built on first use)
+    void *d_radial = nullptr;         // radial-order columns, bin starts and entries (built on first use)
+    size_t radial_start = 0, radial_entries = 0;   // byte offsets of the last two
+    std::vector<int> radial_count;    // offsets per bin
+    int cus = 0;                      // compute units of the device (set with the radial tables)
     StencilOff *d_stencil = nullptr;  // potential / field offsets (rebuilt when the cutoff changes)
     int stencil_kind = -1, stencil_n = 0;  // -1 none, 0 potential, c > 0 field with cutoff c
     double *d_obs = nullptr;          // observable output staging
     size_t obs_cap = 0;
-    int *d_radial_bins = nullptr;
-    std::vector<int> radial_bins;
     unsigned *d_sweep = nullptr;
     unsigned long long *d_counters = nullptr;   // 2 per tile (accepted, rejected)
     std::vector<unsigned long long> replay_counts;  // 2 per replica, from sn_mc_replay
@@ -921,7 +923,7 @@ int sn_destroy(sn_ctx *c)
     void *bufs[] = {c->d_lat, c->d_reps, c->d_tiles, c->d_shapes, c->d_sites,
                     c->d_field_steps, c->d_tile_coord, c->d_gsteps, c->d_pairs,
                     c->d_offs, c->d_sweep,
-                    c->d_counters, c->d_partials, c->d_result, c->d_radial, c->d_radial_bins,
+                    c->d_counters, c->d_partials, c->d_result, c->d_radial,
                     c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
                     c->d_torus_sites, c->d_torus_own[0], c->d_torus_own[1], c->d_torus_near[0],
                     c->d_torus_near[1], c->d_torus_chunks, c->d_rep_counters, c->d_stage};
@@ -1586,32 +1588,77 @@ int sn_moment(sn_ctx *c, int32_t r, double M[3])
     return SN_OK;
 }
 
-// Offsets of radial_order_parameter (src/starrynight-analysis.c:552-561): every
-// (dx,dy,dz) in [-9,9]^3 with r^2 <= 80, grouped by r^2; n = r/|r| in FP64.
-// The reference's r^2 = 81 bin is accumulated but never zeroed or printed
-// (its arrays hold 82 entries, its loops run to 80), so it is left out.
+// Columns of radial_order_parameter (src/starrynight-analysis.c:552-561): half
+// of the (dx, dy) with dx^2 + dy^2 <= 80, near ones first, and for each r^2 the
+// (|dz|, column) that belong to it.  radial_count[b] counts the offsets (dx,
+// dy, dz) of bin b.  The reference's r^2 = 81 bin is accumulated but never
+// zeroed or printed (its arrays hold 82 entries, its loops run to 80), so it
+// is left out.
 static int ensure_radial(sn_ctx *c)
 {
     if (c->d_radial) return SN_OK;
-    std::vector<RadialOff> offs;
+    std::vector<RadialCol> cols;
+    for (int rho2 = 0; rho2 < kRadialBins; rho2++)
+        for (int dx = 0; dx <= kRadialH; dx++)
+            for (int dy = dx ? -kRadialH : 0; dy <= kRadialH; dy++) {
+                if (dx * dx + dy * dy != rho2) continue;
+                const double d = std::sqrt((double)rho2);
+                cols.push_back(rho2 ? RadialCol{dx / d, dy / d, dx, dy} : RadialCol{1.0, 0.0, 0, 0});
+            }
+    const int ncols = (int)cols.size();
+    if (ncols > kRadialCols) return fail(c, SN_ERR_INVALID, "radial columns exceed the table");
+    cols.resize(kRadialCols, cols[0]);
+    std::vector<unsigned short> entries;
     std::vector<int> start(kRadialBins + 1, 0);
+    c->radial_count.assign(kRadialBins, 0);
     for (int b = 0; b < kRadialBins; b++) {
-        start[b] = (int)offs.size();
-        for (int dx = -9; dx <= 9; dx++)
-            for (int dy = -9; dy <= 9; dy++)
-                for (int dz = -9; dz <= 9; dz++) {
-                    if (dx * dx + dy * dy + dz * dz != b) continue;
-                    double d = b ? std::sqrt((double)b) : 1.0;
-                    offs.push_back(RadialOff{dx, dy, dz, 0, dx / d, dy / d, dz / d, 0.0});
-                }
+        start[b] = (int)entries.size();
+        for (int i = 0; i < ncols; i++)
+            for (int k = 0; k <= kRadialH; k++) {
+                const int rho2 = cols[i].dx * cols[i].dx + cols[i].dy * cols[i].dy;
+                if (rho2 + k * k != b) continue;
+                if (i >= 64 && k > kRadialFar) return fail(c, SN_ERR_INVALID, "radial column order");
+                entries.push_back((unsigned short)(k * kRadialCols + i));
+                c->radial_count[b] += (rho2 ? 2 : 1) * (k ? 2 : 1);
+            }
     }
-    start[kRadialBins] = (int)offs.size();
-    HIPCHK(c, hipMalloc((void **)&c->d_radial, offs.size() * sizeof(RadialOff)));
-    HIPCHK(c, hipMalloc((void **)&c->d_radial_bins, start.size() * sizeof(int)));
-    HIPCHK(c, hipMemcpy(c->d_radial, offs.data(), offs.size() * sizeof(RadialOff), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->d_radial_bins, start.data(), start.size() * sizeof(int), hipMemcpyHostToDevice));
-    c->radial_bins = start;
+    start[kRadialBins] = (int)entries.size();
+    HIPCHK(c, hipFuncSetAttribute((const void *)radial_order_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  kRadialLds));
+    HIPCHK(c, hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    // one allocation: columns, bin starts, entries
+    const size_t at_start = cols.size() * sizeof(RadialCol), at_entries = at_start + start.size() * sizeof(int);
+    std::vector<char> table(at_entries + entries.size() * sizeof(unsigned short));
+    std::memcpy(table.data(), cols.data(), at_start);
+    std::memcpy(table.data() + at_start, start.data(), start.size() * sizeof(int));
+    std::memcpy(table.data() + at_entries, entries.data(), entries.size() * sizeof(unsigned short));
+    char *dev = nullptr;
+    HIPCHK(c, hipMalloc((void **)&dev, table.size()));
+    c->d_radial = dev;
+    c->radial_start = at_start;
+    c->radial_entries = at_entries;
+    HIPCHK(c, hipMemcpy(dev, table.data(), table.size(), hipMemcpyHostToDevice));
     return SN_OK;
+}
+
+// Workgroups of 4 rows x tz sites, each over a range of x.  A workgroup stages
+// eight planes before its first, so the ranges are as long as the rounds over
+// the chip allow: the fewest (workgroups per CU) x (planes computed + a
+// quarter of the planes staged before; a plane's loads took about that).
+static void radial_split(const RepHost &h, int cus, int &ny, int &nz, int &tz, int &cx)
+{
+    ny = (h.Y + kRadialTY - 1) / kRadialTY;
+    nz = (h.Z + kRadialTZ - 1) / kRadialTZ;
+    tz = (h.Z + nz - 1) / nz;
+    const long long columns = (long long)ny * nz;
+    double best = 0.0;
+    cx = h.X;
+    for (int parts = 1; parts <= h.X; parts++) {
+        const int len = (h.X + parts - 1) / parts;
+        const long long rounds = (columns * parts + cus - 1) / cus;
+        const double cost = (double)rounds * (len + 0.25 * kRadialH);
+        if (parts == 1 || cost < best) { best = cost; cx = len; }
+    }
 }
 
 int sn_radial_order(sn_ctx *c, int32_t r, double fe[81], double afe[81], int64_t count[81])
@@ -1621,10 +1668,15 @@ int sn_radial_order(sn_ctx *c, int32_t r, double fe[81], double afe[81], int64_t
     if (!fe || !afe || !count) return fail(c, SN_ERR_INVALID, "null output");
     if ((st = ensure_radial(c))) return st;
     const RepHost &h = c->reps[r];
-    int nblk = (int)std::min<long long>((h.N + 255) / 256, 2048);
+    int ny, nz, tz, cx;
+    radial_split(h, c->cus, ny, nz, tz, cx);
+    const int nblk = ny * nz * ((h.X + cx - 1) / cx);
     if ((st = ensure_partials(c, (size_t)nblk * 2 * kRadialBins))) return st;
-    hipLaunchKernelGGL(radial_order_kernel, dim3(nblk), dim3(256), 0, c->stream, c->d_lat, c->d_reps, r,
-                       c->d_radial, c->d_radial_bins, c->d_partials);
+    const char *table = (const char *)c->d_radial;
+    RadialArgs ra{c->d_lat, c->d_reps, (const RadialCol *)table,
+                  (const unsigned short *)(table + c->radial_entries), (const int *)(table + c->radial_start),
+                  c->d_partials, r, ny, nz, tz, cx};
+    hipLaunchKernelGGL(radial_order_kernel, dim3(nblk), dim3(kRadialThreads), kRadialLds, c->stream, ra);
     HIPCHK(c, hipGetLastError());
     launch_reduce(c, nblk, 2 * kRadialBins);
     HIPCHK(c, hipGetLastError());
@@ -1632,7 +1684,7 @@ int sn_radial_order(sn_ctx *c, int32_t r, double fe[81], double afe[81], int64_t
     double sums[2 * kRadialBins];
     HIPCHK(c, hipMemcpy(sums, c->d_result, sizeof(sums), hipMemcpyDeviceToHost));
     for (int b = 0; b < kRadialBins; b++) {
-        const long long cnt = h.N * (long long)(c->radial_bins[b + 1] - c->radial_bins[b]);
+        const long long cnt = h.N * (long long)c->radial_count[b];
         count[b] = cnt;
         fe[b] = cnt ? sums[2 * b] / (double)cnt : 0.0;
         afe[b] = cnt ? sums[2 * b + 1] / (double)cnt : 0.0;

@@ -1,0 +1,29 @@
+"""Observable kernels at the edges of their tiles, against the oracle.
+
+Bars as in test_gpu_energy: FP64 on both sides, only the summation order
+differs; counts exact.
+"""
+import numpy as np
+import pytest
+
+from tests.helpers import oracle_model, print_case, rand_lattice
+
+pytestmark = pytest.mark.gpu
+
+# workgroups of 4 rows x up to 16 z walk along x over a ring of ten planes:
+# rows left over, z split unevenly, one plane, more planes than the ring has,
+# every axis shorter than the reach of 8 sites
+RADIAL = [(2, 2, 1), (2, 3, 2), (2, 5, 17), (9, 4, 16), (23, 6, 33), (64, 2, 3), (31, 7, 1)]
+
+
+@pytest.mark.parametrize("dims", RADIAL)
+def test_radial_order_tiles(sn, oracle, dims):
+    rp = sn.ReplicaParams(*dims, DipoleCutOff=1)
+    print_case("radial_tiles", dims=dims)
+    lat = rand_lattice(rp.N, np.random.default_rng(sum(dims)), mixed=True)
+    with sn.StarryNight(rp) as ctx:
+        ctx.set_lattice(lat)
+        fe, afe, cnt = ctx.radial_order()
+    few, afew, cntw = oracle_model(oracle, rp).radial_order(lat)
+    assert np.array_equal(cnt, cntw)
+    assert np.abs(fe - few).max() <= 1e-12 and np.abs(afe - afew).max() <= 1e-12
