@@ -14,6 +14,7 @@
 #include "../../include/starrynight_amd.h"
 #include "sn_aux_kernels.h"
 #include "sn_radial.h"
+#include "sn_stencil.h"
 #include "sn_dispatch.h"
 #include "sn_schedule.h"
 
@@ -70,8 +71,7 @@ struct sn_ctx {
     size_t radial_start = 0, radial_entries = 0;   // byte offsets of the last two
     std::vector<int> radial_count;    // offsets per bin
     int cus = 0;                      // compute units of the device (set with the radial tables)
-    StencilOff *d_stencil = nullptr;  // potential / field offsets (rebuilt when the cutoff changes)
-    int stencil_kind = -1, stencil_n = 0;  // -1 none, 0 potential, c > 0 field with cutoff c
+    double *d_stencil[kFieldMaxR + 1] = {};   // weights: 0 potential, c > 0 field of cutoff c (built on first use)
     double *d_obs = nullptr;          // observable output staging
     size_t obs_cap = 0;
     unsigned *d_sweep = nullptr;
@@ -924,11 +924,13 @@ int sn_destroy(sn_ctx *c)
                     c->d_field_steps, c->d_tile_coord, c->d_gsteps, c->d_pairs,
                     c->d_offs, c->d_sweep,
                     c->d_counters, c->d_partials, c->d_result, c->d_radial,
-                    c->d_stencil, c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
+                    c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
                     c->d_torus_sites, c->d_torus_own[0], c->d_torus_own[1], c->d_torus_near[0],
                     c->d_torus_near[1], c->d_torus_chunks, c->d_rep_counters, c->d_stage};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    for (double *w : c->d_stencil)
+        if (w) (void)hipFree(w);
     if (c->h_result) (void)hipHostFree(c->h_result);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1692,33 +1694,48 @@ int sn_radial_order(sn_ctx *c, int32_t r, double fe[81], double afe[81], int64_t
     return SN_OK;
 }
 
-// Offsets of dipole_potential (kind 0: 0 < |r| <= 6, src/starrynight-analysis.c:72-80)
-// or dipole_electricfield (kind = cutoff: 0 < |r| <= cutoff, :403-413), in the
-// reference's dx, dy, dz loop order; the dz range runs when Z == 1.
+typedef void (*StencilFn)(StencilArgs);
+static StencilFn pick_stencil(int kind)
+{
+    switch (kind) {
+    case 0: return stencil_observable_kernel<kPotentialR, false, stencil_nx(kPotentialR, false)>;
+#define SN_FIELD(r) case r: return stencil_observable_kernel<r, true, stencil_nx(r, true)>;
+    SN_FIELD(1) SN_FIELD(2) SN_FIELD(3) SN_FIELD(4) SN_FIELD(5) SN_FIELD(6) SN_FIELD(7) SN_FIELD(8) SN_FIELD(9)
+#undef SN_FIELD
+    }
+    return nullptr;
+}
+
+// Weights of dipole_potential (kind 0: 0 < |r| <= 6, src/starrynight-analysis.c:72-80)
+// or dipole_electricfield (kind = cutoff: 0 < |r| <= cutoff, :403-413), one
+// table per kind, kept by the context; the dz range runs when Z == 1.
 static int ensure_stencil(sn_ctx *c, int kind)
 {
-    if (c->d_stencil && c->stencil_kind == kind) return SN_OK;
-    const int R = kind == 0 ? 6 : kind;
-    std::vector<StencilOff> offs;
-    for (int dx = -R; dx <= R; dx++)
-        for (int dy = -R; dy <= R; dy++)
-            for (int dz = -R; dz <= R; dz++) {
+    if (c->d_stencil[kind]) return SN_OK;
+    const int R = kind == 0 ? kPotentialR : kind;
+    const int row = stencil_row(R, kind != 0);
+    std::vector<double> weights(stencil_weights(R, kind != 0), 0.0);
+    for (int dx = 0; dx <= R; dx++)
+        for (int dy = 0; dy <= R; dy++)
+            for (int dz = 0; dz <= R; dz++) {
                 const int d2 = dx * dx + dy * dy + dz * dz;
                 if (d2 == 0 || d2 > R * R) continue;
-                const double d = std::sqrt((double)d2), w = 1.0 / (d * d * d);
-                if (kind == 0) offs.push_back(StencilOff{dx, dy, dz, 0, dx * w, dy * w, dz * w, w});
-                else offs.push_back(StencilOff{dx, dy, dz, 0, dx / d, dy / d, dz / d, w});
+                const double d = std::sqrt((double)d2);
+                double *w = &weights[(size_t)(dx * (R + 1) + dy) * row + dz];
+                w[0] = 1.0 / (d * d * d);
+                if (kind) w[R + 1] = 3.0 / (d * d * d * d2);
             }
-    if (c->d_stencil) (void)hipFree(c->d_stencil);
-    c->d_stencil = nullptr;
-    HIPCHK(c, hipMalloc((void **)&c->d_stencil, offs.size() * sizeof(StencilOff)));
-    HIPCHK(c, hipMemcpy(c->d_stencil, offs.data(), offs.size() * sizeof(StencilOff), hipMemcpyHostToDevice));
-    c->stencil_kind = kind;
-    c->stencil_n = (int)offs.size();
+    HIPCHK(c, hipFuncSetAttribute((const void *)pick_stencil(kind), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)stencil_lds(R)));
+    double *dev = nullptr;
+    HIPCHK(c, hipMalloc((void **)&dev, weights.size() * sizeof(double)));
+    c->d_stencil[kind] = dev;
+    HIPCHK(c, hipMemcpy(dev, weights.data(), weights.size() * sizeof(double), hipMemcpyHostToDevice));
     return SN_OK;
 }
 
-static int run_stencil(sn_ctx *c, int32_t r, int kind, double *host_out, int width)
+// Launches the stencil of `kind` into d_obs (width values per site).
+static int launch_stencil(sn_ctx *c, int32_t r, int kind, int width)
 {
     const RepHost &h = c->reps[r];
     int st;
@@ -1727,19 +1744,27 @@ static int run_stencil(sn_ctx *c, int32_t r, int kind, double *host_out, int wid
     if (need > c->obs_cap) {
         if (c->d_obs) (void)hipFree(c->d_obs);
         c->d_obs = nullptr;
+        c->obs_cap = 0;
         HIPCHK(c, hipMalloc((void **)&c->d_obs, need * sizeof(double)));
         c->obs_cap = need;
     }
-    const unsigned nb = (unsigned)((h.N + 255) / 256);
-    if (kind == 0)
-        hipLaunchKernelGGL(stencil_observable_kernel<false>, dim3(nb), dim3(256), 0, c->stream, c->d_lat, c->d_reps,
-                           r, c->d_stencil, c->stencil_n, c->d_obs);
-    else
-        hipLaunchKernelGGL(stencil_observable_kernel<true>, dim3(nb), dim3(256), 0, c->stream, c->d_lat, c->d_reps,
-                           r, c->d_stencil, c->stencil_n, c->d_obs);
+    const int R = kind == 0 ? kPotentialR : kind, nx = stencil_nx(R, kind != 0);
+    const bool whole = h.Z <= 64;
+    const int zl = whole ? h.Z : 64, rows = 64 / zl, valid = whole ? h.Z : 64 - 2 * R;
+    const int ny = (h.Y + 8 * rows - 1) / (8 * rows), nz = (h.Z + valid - 1) / valid;
+    StencilArgs sa{c->d_lat, c->d_reps, c->d_stencil[kind], c->d_obs, r, ny, nz, zl, rows, valid};
+    hipLaunchKernelGGL(pick_stencil(kind), dim3((unsigned)(ny * nz * ((h.X + nx - 1) / nx))), dim3(kStencilThreads),
+                       stencil_lds(R), c->stream, sa);
     HIPCHK(c, hipGetLastError());
+    return SN_OK;
+}
+
+static int run_stencil(sn_ctx *c, int32_t r, int kind, double *host_out, int width)
+{
+    int st;
+    if ((st = launch_stencil(c, r, kind, width))) return st;
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(host_out, c->d_obs, need * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHK(c, hipMemcpy(host_out, c->d_obs, (size_t)c->reps[r].N * width * sizeof(double), hipMemcpyDeviceToHost));
     return SN_OK;
 }
 
@@ -1756,7 +1781,7 @@ int sn_dipole_efield(sn_ctx *c, int32_t r, int32_t cutoff, double *E)
     int st = check_rep(c, r);
     if (st) return st;
     if (!E) return fail(c, SN_ERR_INVALID, "null output");
-    if (cutoff < 1 || cutoff > 9) return fail(c, SN_ERR_RANGE, "field cutoff must be in 1..9");
+    if (cutoff < 1 || cutoff > kFieldMaxR) return fail(c, SN_ERR_RANGE, "field cutoff must be in 1..9");
     return run_stencil(c, r, cutoff, E, 3);
 }
 
@@ -1766,8 +1791,7 @@ int sn_recombination(sn_ctx *c, int32_t r, double out[8])
     if (st) return st;
     if (!out) return fail(c, SN_ERR_INVALID, "null output");
     const RepHost &h = c->reps[r];
-    std::vector<double> pot(h.N);
-    if ((st = run_stencil(c, r, 0, pot.data(), 1))) return st;   // leaves the potential in d_obs
+    if ((st = launch_stencil(c, r, 0, 1))) return st;   // the potential, in d_obs
     const int nblk = (int)std::min<long long>((h.N + 255) / 256, 1024);
     if ((st = ensure_partials(c, (size_t)nblk * kRecombParts))) return st;
     // the reference's constants: 0.165 eV per internal unit, screened by 5; kT = 0.025 eV

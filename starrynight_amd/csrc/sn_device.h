@@ -213,6 +213,20 @@ __device__ __forceinline__ int wrap_once(int v, int L)
     return v;
 }
 
+__device__ __forceinline__ int wrap_any(int v, int L)
+{
+    const int m = v % L;
+    return m < 0 ? m + L : m;
+}
+
+// Consecutive workgroups go to the eight XCDs in turn; this numbering gives
+// each XCD (each L2) a contiguous eighth of the work instead.
+__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n)
+{
+    const unsigned xcd = b % 8, each = n / 8, rest = n % 8;
+    return xcd * each + min(xcd, rest) + b / 8;
+}
+
 template <int G>
 __device__ __forceinline__ double group_sum(double v)
 {

@@ -119,12 +119,6 @@ __device__ __forceinline__ void radial_row(const double *a, const double *q, int
     radial_steps(step, n, std::make_integer_sequence<int, kRadialTZ>());
 }
 
-__device__ __forceinline__ int wrap_any(int v, int n)
-{
-    const int m = v % n;
-    return m < 0 ? m + n : m;
-}
-
 __global__ __launch_bounds__(kRadialThreads) void radial_order_kernel(RadialArgs ra)
 {
     extern __shared__ double lds[];
@@ -133,7 +127,8 @@ __global__ __launch_bounds__(kRadialThreads) void radial_order_kernel(RadialArgs
     const bool far = wave >= kRadialTY;
     const RepDev &rep = ra.reps[ra.replica];
     const int X = rep.X, Y = rep.Y, Z = rep.Z;
-    const int z0 = (int)(blockIdx.x % ra.nz) * ra.tz, q0 = (int)blockIdx.x / ra.nz;
+    const int block = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int z0 = block % ra.nz * ra.tz, q0 = block / ra.nz;
     const int y0 = q0 % ra.ny * kRadialTY, x0 = q0 / ra.ny * ra.cx;
     const int n = min(ra.tz, Z - z0);
     const int x1 = min(x0 + ra.cx, X);
@@ -220,7 +215,7 @@ __global__ __launch_bounds__(kRadialThreads) void radial_order_kernel(RadialArgs
             for (int r = 0; r < kRadialTY; r++) t += o[2 * r * kRadialSums];
             s += t;
         }
-        ra.partials[(long long)blockIdx.x * 2 * kRadialBins + tid] = s;
+        ra.partials[(long long)block * 2 * kRadialBins + tid] = s;
     }
 }
 

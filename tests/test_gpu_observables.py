@@ -27,3 +27,21 @@ def test_radial_order_tiles(sn, oracle, dims):
     few, afew, cntw = oracle_model(oracle, rp).radial_order(lat)
     assert np.array_equal(cnt, cntw)
     assert np.abs(fe - few).max() <= 1e-12 and np.abs(afe - afew).max() <= 1e-12
+
+
+# rows held whole by the lanes (several to a wave below 33 sites) and cut at
+# Z > 64; rows of a workgroup left over; an odd X; axes shorter than the reach
+STENCIL = [(2, 3, 2), (5, 70, 1), (3, 9, 31), (4, 17, 64), (3, 5, 65), (7, 4, 130)]
+
+
+@pytest.mark.parametrize("dims", STENCIL)
+def test_stencil_tiles(sn, oracle, dims):
+    rp = sn.ReplicaParams(*dims, DipoleCutOff=1)
+    print_case("stencil_tiles", dims=dims)
+    lat = rand_lattice(rp.N, np.random.default_rng(sum(dims)), mixed=True)
+    o = oracle_model(oracle, rp)
+    with sn.StarryNight(rp) as ctx:
+        ctx.set_lattice(lat)
+        assert np.abs(ctx.dipole_potential() - o.dipole_potential(lat)).max() <= 1e-12
+        for cutoff in range(1, 10):
+            assert np.abs(ctx.dipole_efield(cutoff) - o.dipole_efield(lat, cutoff)).max() <= 1e-12
