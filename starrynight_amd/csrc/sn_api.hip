@@ -1082,8 +1082,9 @@ int sn_site_energy_batch_device(sn_ctx *c, int32_t r, int64_t n, const int32_t *
     if (n < 0) return fail(c, SN_ERR_INVALID, "negative count");
     if (n == 0) return SN_OK;
     if (!site || !prop || !dE) return fail(c, SN_ERR_INVALID, "null buffer");
-    long long nb = (n + 255) / 256;
-    hipLaunchKernelGGL(site_energy_batch_kernel, dim3((unsigned)nb), dim3(256), 0, c->stream, c->d_lat,
+    const long long per_block = kMoveThreads / kMoveLanes;
+    const unsigned nb = (unsigned)std::min<long long>((n + per_block - 1) / per_block, kMoveBlocks);
+    hipLaunchKernelGGL(site_energy_batch_kernel, dim3(nb), dim3(kMoveThreads), move_lds(c->noff), c->stream, c->d_lat,
                        c->d_reps, r, c->d_offs, c->noff, (long long)n, site, prop, dE);
     HIPCHK(c, hipGetLastError());
     return SN_OK;
