@@ -29,6 +29,14 @@ struct RepHost {
     double L0;
 };
 
+// Workgroups of the energy kernel, grouped by replica.
+struct EnergyList {
+    EnergyBlock *blocks = nullptr;
+    int *seg = nullptr;              // off on the device
+    std::vector<int> off;            // R + 1 offsets into blocks
+    std::vector<char> wide;          // per replica: energy_wide successive x per workgroup, else one
+};
+
 }  // namespace
 
 // Partial sums of sn_gradient_all_device_noalloc: a fixed device array, one
@@ -87,10 +95,9 @@ struct sn_ctx {
     double *d_scratch = nullptr;   // this device's `scratch` array (not owned)
     int gather_region = 0;   // largest staged region of the gather kernel (z rows padded, gather_zstride)
     int field_region = 0;   // largest staged region of the field kernel (z rows padded to odd)
-    int *d_tile_list = nullptr;          // tile indices grouped by replica (tiled energy kernel)
-    int *d_tile_seg = nullptr;           // R + 1 offsets into d_tile_list (device copy)
+    EnergyList energy_all, energy_each;  // workgroups of the energy kernel: all replicas in one launch, one replica
     double *h_result = nullptr;          // pinned host copy of d_result
-    std::vector<int> rep_tile_off;       // R + 1 offsets into d_tile_list
+    std::vector<int> rep_tiles;          // tiles per replica
     bool energy_tiled = false;           // energy / gradient through tile_energy_kernel
     // whole-lattice sweeps of small replicas (kernel 3): one workgroup per replica
     bool torus = false;
@@ -208,6 +215,72 @@ static int ensure_stage(sn_ctx *c, size_t bytes)
     HIPCHK(c, hipMalloc(&c->d_stage, cap));
     c->stage_cap = cap;
     return SN_OK;
+}
+
+// Workgroups of the energy kernel for one launch over all replicas (together)
+// or for a launch per replica.
+static int energy_list(sn_ctx *c, bool together, EnergyList &list)
+{
+    const int nx_wide = energy_wide(c->rc, c->two_d), rc = c->rc;
+    struct Split { int zl, nz, valid, ny, rows; };
+    std::vector<Split> split(c->R);
+    constexpr int kCUs = 256;
+    for (int r = 0; r < c->R; r++) {
+        const RepHost &h = c->reps[r];
+        // the cut of a row into nz (1: whole, no halo) that leaves the fewest
+        // workgroups, of rows whose staged plane fits
+        Split &p = split[r];
+        p.ny = 0;
+        for (int nz = 1; nz <= h.Z; nz++) {
+            const int valid = (h.Z + nz - 1) / nz, zl = nz == 1 ? valid : valid + 2 * rc;
+            const int most = std::min(kEnergyThreads / zl, kEnergyRegion / zl - 2 * rc);
+            if (most < 1) continue;
+            const int ny = (h.Y + most - 1) / most;
+            if (p.ny && ny * nz >= p.ny * p.nz) {
+                if (zl < 32) break;
+                continue;
+            }
+            p = Split{zl, nz, valid, ny, (h.Y + ny - 1) / ny};
+        }
+    }
+    // x per step (one or nx_wide) and steps per workgroup: the fewest rounds
+    // over the chip, times a workgroup's planes.  A step costs its planes and
+    // an exchange per output, of about a plane; a workgroup's start and end
+    // cost about six planes; a CU holds one.  48^3 alone takes one x a step in
+    // 240 workgroups (14 us), 64^3 two in 256 (15 us; one a step 19 us).
+    auto choose = [&](int r0, int r1, int &nx, int &len) {
+        int longest = 0;
+        for (int r = r0; r < r1; r++) longest = std::max(longest, c->reps[r].X);
+        double best = -1.0;
+        for (int step : {1, nx_wide})
+            for (int steps = 1; (steps - 1) * step < longest; steps++) {
+                long long blocks = 0;
+                for (int r = r0; r < r1; r++)
+                    blocks += (long long)((c->reps[r].X + step * steps - 1) / (step * steps)) * split[r].ny * split[r].nz;
+                const double cost = (double)((blocks + kCUs - 1) / kCUs) * (steps * (2 * rc + 2 * step) + 6);
+                if (best < 0.0 || cost < best) { best = cost; nx = step; len = step * steps; }
+            }
+    };
+    int nx = 1, len = 1;
+    if (together) choose(0, c->R, nx, len);
+    std::vector<EnergyBlock> blocks;
+    list.off.assign(1, 0);
+    list.wide.assign(c->R, 0);
+    for (int r = 0; r < c->R; r++) {
+        const RepHost &h = c->reps[r];
+        const Split &p = split[r];
+        if (!together) choose(r, r + 1, nx, len);
+        list.wide[r] = nx == nx_wide;
+        for (int x = 0; x < h.X; x += len)
+            for (int y = 0; y < h.Y; y += p.rows)
+                for (int k = 0; k < p.nz; k++)
+                    blocks.push_back(EnergyBlock{r, x, std::min(len, h.X - x), y, std::min(p.rows, h.Y - y), k * p.valid,
+                                                 p.zl, 0});
+        list.off.push_back((int)blocks.size());
+    }
+    int st;
+    if ((st = upload(c, &list.blocks, blocks))) return st;
+    return upload(c, &list.seg, list.off);
 }
 
 // Byte offsets of consecutive 256-byte-aligned slices of the staging buffer.
@@ -888,22 +961,15 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
         else c->err = keep;
     }
     if (!tiles_ok) return SN_OK;
-    // the tiled energy kernel stages the field kernel's padded region
-    const size_t energy_lds = (size_t)4 * field_region_doubles(c) * sizeof(double);
-    if (pick_energy(c->rc, c->two_d, false) && energy_lds <= 150 * 1024) {
-        std::vector<int> tl;
-        c->rep_tile_off.assign(c->R + 1, 0);
-        for (int r = 0; r < c->R; r++) {
-            c->rep_tile_off[r] = (int)tl.size();
-            for (size_t t = 0; t < c->sched.tiles.size(); t++)
-                if (c->sched.tiles[t].replica == r) tl.push_back((int)t);
-        }
-        c->rep_tile_off[c->R] = (int)tl.size();
-        if ((st = upload(c, &c->d_tile_list, tl))) return st;
-        if ((st = upload(c, &c->d_tile_seg, c->rep_tile_off))) return st;
-        for (int m = 0; m < 2; m++)
-            HIPCHK(c, hipFuncSetAttribute((const void *)pick_energy(c->rc, c->two_d, m == 1),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)energy_lds));
+    // (cut-offs whose tiles the energy kernel was first built on)
+    if (pick_energy(c->rc, c->two_d, false, false) && (size_t)4 * field_region_doubles(c) * sizeof(double) <= 150 * 1024) {
+        c->rep_tiles.assign(c->R, 0);
+        for (const Tile &t : c->sched.tiles) c->rep_tiles[t.replica]++;
+        if ((st = energy_list(c, true, c->energy_all)) || (st = energy_list(c, false, c->energy_each))) return st;
+        for (int m = 0; m < 4; m++)
+            HIPCHK(c, hipFuncSetAttribute((const void *)pick_energy(c->rc, c->two_d, m & 1, m & 2),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          (int)energy_lds(c->two_d, m & 1)));
         c->energy_tiled = true;
     }
     for (int m = 0; m < 2; m++) {
@@ -924,7 +990,8 @@ int sn_destroy(sn_ctx *c)
                     c->d_field_steps, c->d_tile_coord, c->d_gsteps, c->d_pairs,
                     c->d_offs, c->d_sweep,
                     c->d_counters, c->d_partials, c->d_result, c->d_radial,
-                    c->d_obs, c->d_tile_list, c->d_tile_seg, c->d_torus_box_of, c->d_torus_boxes,
+                    c->d_obs, c->energy_all.blocks, c->energy_all.seg, c->energy_each.blocks,
+                    c->energy_each.seg, c->d_torus_box_of, c->d_torus_boxes,
                     c->d_torus_sites, c->d_torus_own[0], c->d_torus_own[1], c->d_torus_near[0],
                     c->d_torus_near[1], c->d_torus_chunks, c->d_rep_counters, c->d_stage};
     for (void *b : bufs)
@@ -1445,24 +1512,33 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
     };
     double *part = nullptr;
     if (c->energy_tiled) {
-        const int t0 = all ? 0 : c->rep_tile_off[r], t1 = all ? c->rep_tile_off[c->R] : c->rep_tile_off[r + 1];
-        const int nblk = t1 - t0;
-        if ((st = partials((size_t)nblk * kNPart, &part))) return st;
-        // one launch: the mixed-length variant serves uniform replicas too
-        const bool mixed = all ? any_mixed(c) : c->reps[r].mixed != 0;
-        EnergyArgs ea;
-        ea.lat = c->d_lat; ea.reps = c->d_reps; ea.tiles = c->d_tiles; ea.shapes = c->d_shapes;
-        ea.tile_list = c->d_tile_list + t0;
-        ea.grad = dg; ea.grad_origin = all ? 0 : c->reps[r].base;
-        ea.partials = part;
-        ea.region_doubles = field_region_doubles(c);
-        const size_t lds = (size_t)(mixed ? 4 : 3) * ea.region_doubles * sizeof(double);
-        hipLaunchKernelGGL(pick_energy(c->rc, c->two_d, mixed), dim3(nblk), dim3(kBlock), lds, c->stream, ea);
-        HIPCHK(c, hipGetLastError());
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3((kNPart + kReduceCols - 1) / kReduceCols, all ? c->R : 1),
-                           dim3(256), 0, c->stream, part, nblk, kNPart, c->d_result,
-                           all ? (const int *)c->d_tile_seg : (const int *)nullptr);
-        HIPCHK(c, hipGetLastError());
+        int tiles = 0;
+        for (int q = all ? 0 : r; q < (all ? c->R : r + 1); q++) tiles += c->rep_tiles[q];
+        if (fixed_partials && (st = partials((size_t)tiles * kNPart, &part))) return st;   // (a row per tile)
+        // one launch over replicas q0..q1-1, whose sums go to d_result + out * kNPart
+        auto launch = [&](const EnergyList &list, int q0, int q1, bool mixed, double *g, int out) -> int {
+            const int nblk = list.off[q1] - list.off[q0];
+            int e;
+            if ((e = partials((size_t)nblk * kNPart, &part))) return e;
+            EnergyArgs ea{c->d_lat, c->d_reps, list.blocks + list.off[q0], g, q1 - q0 > 1 || all ? 0 : c->reps[q0].base,
+                          part};
+            hipLaunchKernelGGL(pick_energy(c->rc, c->two_d, mixed, list.wide[q0]), dim3(nblk), dim3(kEnergyThreads),
+                               energy_lds(c->two_d, mixed), c->stream, ea);
+            HIPCHK(c, hipGetLastError());
+            hipLaunchKernelGGL(reduce_partials_kernel, dim3((kNPart + kReduceCols - 1) / kReduceCols, q1 - q0),
+                               dim3(256), 0, c->stream, part, nblk, kNPart, c->d_result + out * kNPart,
+                               q1 - q0 > 1 ? (const int *)list.seg : (const int *)nullptr);
+            HIPCHK(c, hipGetLastError());
+            return SN_OK;
+        };
+        if (!all) return launch(c->energy_each, r, r + 1, c->reps[r].mixed != 0, dg, 0);
+        // one launch (the mixed-length variant serves uniform replicas too),
+        // or, where the fixed scratch holds a row per tile but not one per
+        // workgroup, a launch per replica: they use it in stream order
+        if (!fixed_partials || (size_t)c->energy_all.off[c->R] * kNPart <= fixed_cap)
+            return launch(c->energy_all, 0, c->R, any_mixed(c), dg, 0);
+        for (int q = 0; q < c->R; q++)
+            if ((st = launch(c->energy_each, q, q + 1, c->reps[q].mixed != 0, dg, q))) return st;
         return SN_OK;
     }
     // per-site gather kernel, one replica at a time (the partials buffer is

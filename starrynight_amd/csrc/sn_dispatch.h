@@ -2,7 +2,7 @@
 // template instances are compiled in their own translation units
 // (sn_gather_kernels.hip, sn_field_kernels_rc*.hip) so the build runs in parallel.
 #pragma once
-#include "sn_energy_tiled.h"
+#include "sn_energy.h"
 #include "sn_torus.h"
 #include "sn_sweep_field.h"
 
@@ -35,12 +35,26 @@ FieldFn pick_field_rc4(bool two_d, bool mixed);
 FieldFn pick_field_rc5(bool two_d, bool mixed);
 
 typedef void (*EnergyFn)(EnergyArgs);
-// tiled energy / adjoint kernel for DipoleCutOff rc (1..5) or null
-EnergyFn pick_energy(int rc, bool two_d, bool mixed);
-EnergyFn pick_energy_rc1(bool two_d, bool mixed);
-EnergyFn pick_energy_rc2(bool two_d, bool mixed);
-EnergyFn pick_energy_rc3(bool two_d, bool mixed);
-EnergyFn pick_energy_rc4(bool two_d, bool mixed);
-EnergyFn pick_energy_rc5(bool two_d, bool mixed);
+// energy / adjoint kernel for DipoleCutOff rc (1..5) or null; wide: energy_wide
+// successive x per workgroup instead of one
+EnergyFn pick_energy(int rc, bool two_d, bool mixed, bool wide);
+EnergyFn pick_energy_rc1(bool two_d, bool mixed, bool wide);
+EnergyFn pick_energy_rc2(bool two_d, bool mixed, bool wide);
+EnergyFn pick_energy_rc3(bool two_d, bool mixed, bool wide);
+EnergyFn pick_energy_rc4(bool two_d, bool mixed, bool wide);
+EnergyFn pick_energy_rc5(bool two_d, bool mixed, bool wide);
+
+template <int RC, bool TWO_D, bool MIXED>
+EnergyFn energy_instance(bool wide)
+{
+    return wide ? (EnergyFn)energy_kernel<RC, TWO_D, MIXED, energy_wide(RC, TWO_D)>
+                : (EnergyFn)energy_kernel<RC, TWO_D, MIXED, 1>;
+}
+template <int RC>
+EnergyFn energy_instance(bool two_d, bool mixed, bool wide)
+{
+    return two_d ? (mixed ? energy_instance<RC, true, true>(wide) : energy_instance<RC, true, false>(wide))
+                 : (mixed ? energy_instance<RC, false, true>(wide) : energy_instance<RC, false, false>(wide));
+}
 
 }  // namespace sn

@@ -1,4 +1,4 @@
-// sn_field_kernels_rc1.hip -- field-update sweep and tiled energy kernel instances for
+// sn_field_kernels_rc1.hip -- field-update sweep and energy kernel instances for
 // DipoleCutOff = 1.
 #include <hip/hip_runtime.h>
 
@@ -14,12 +14,9 @@ FieldFn pick_field_rc1(bool two_d, bool mixed)
                  : (FieldFn)field_sweep_kernel<1, false, false, kFieldG>;
 }
 
-EnergyFn pick_energy_rc1(bool two_d, bool mixed)
+EnergyFn pick_energy_rc1(bool two_d, bool mixed, bool wide)
 {
-    if (two_d) return mixed ? (EnergyFn)tile_energy_kernel<1, true, true>
-                            : (EnergyFn)tile_energy_kernel<1, true, false>;
-    return mixed ? (EnergyFn)tile_energy_kernel<1, false, true>
-                 : (EnergyFn)tile_energy_kernel<1, false, false>;
+    return energy_instance<1>(two_d, mixed, wide);
 }
 
 }  // namespace sn

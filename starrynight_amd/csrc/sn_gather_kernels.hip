@@ -50,14 +50,14 @@ TorusFn pick_torus(int G, int NPL, bool mixed, int blk, bool two)
     return nullptr;
 }
 
-EnergyFn pick_energy(int rc, bool two_d, bool mixed)
+EnergyFn pick_energy(int rc, bool two_d, bool mixed, bool wide)
 {
     switch (rc) {
-    case 1: return pick_energy_rc1(two_d, mixed);
-    case 2: return pick_energy_rc2(two_d, mixed);
-    case 3: return pick_energy_rc3(two_d, mixed);
-    case 4: return pick_energy_rc4(two_d, mixed);
-    case 5: return pick_energy_rc5(two_d, mixed);
+    case 1: return pick_energy_rc1(two_d, mixed, wide);
+    case 2: return pick_energy_rc2(two_d, mixed, wide);
+    case 3: return pick_energy_rc3(two_d, mixed, wide);
+    case 4: return pick_energy_rc4(two_d, mixed, wide);
+    case 5: return pick_energy_rc5(two_d, mixed, wide);
     }
     return nullptr;
 }

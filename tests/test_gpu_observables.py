@@ -45,3 +45,30 @@ def test_stencil_tiles(sn, oracle, dims):
         assert np.abs(ctx.dipole_potential() - o.dipole_potential(lat)).max() <= 1e-12
         for cutoff in range(1, 10):
             assert np.abs(ctx.dipole_efield(cutoff) - o.dipole_efield(lat, cutoff)).max() <= 1e-12
+
+
+# rows held whole or cut (Z = 180: halo inside the lattice), rows and x left
+# over by the workgroups, workgroups of several steps along x, one and two x a
+# step, plane (2D) lattices of more rows than lanes
+ENERGY = [((8, 7, 6), 3), ((7, 30, 5), 2), ((9, 12, 180), 4), ((10, 9, 70), 1), ((33, 20, 16), 5), ((16, 600, 1), 3),
+          ((300, 10, 1), 5), ((64, 64, 64), 3)]
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("dims,rc", ENERGY)
+def test_energy_workgroups(sn, oracle, dims, rc, mixed):
+    rp = sn.ReplicaParams(*dims, DipoleCutOff=rc, CageStrain=0.7, Efield=(0.01, -0.02, 0.03), K=0.2)
+    print_case("energy_workgroups", dims=dims, rc=rc, mixed=mixed)
+    lat = rand_lattice(rp.N, np.random.default_rng(sum(dims) + rc), mixed=mixed)
+    with sn.StarryNight(rp) as ctx:
+        ctx.set_lattice(lat)
+        e, parts = ctx.energy()
+        g, dp, e2 = ctx.gradient()
+    o = oracle_model(oracle, rp)
+    ew, pw = o.energy(lat)
+    gw, dpw = o.gradient(lat)
+    scale = np.abs(pw).sum() + 1.0
+    assert abs(e - ew) <= 1e-12 * scale and e2 == e
+    assert np.abs(parts - pw).max() <= 1e-12 * scale
+    assert np.abs(g - gw).max() <= 1e-11 * (np.abs(gw).max() + 1.0)
+    assert np.abs(dp - dpw).max() <= 1e-11 * (np.abs(dpw).max() + 1.0)
