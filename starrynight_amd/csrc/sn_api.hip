@@ -313,8 +313,8 @@ struct EventList {
 // doubles), kReduceCols columns per workgroup.
 static void launch_reduce(sn_ctx *c, int nblk, int width)
 {
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3((width + kReduceCols - 1) / kReduceCols), dim3(256), 0,
-                       c->stream, c->d_partials, nblk, width, c->d_result, (const int *)nullptr);
+    hipLaunchKernelGGL(reduce_partials_kernel, dim3((width + kReduceCols - 1) / kReduceCols),
+                       dim3(kReduceThreads), 0, c->stream, c->d_partials, nblk, width, c->d_result, (const int *)nullptr);
 }
 
 // Largest tile + halo (sites) staged in LDS: 4 doubles per site (mixed lengths)
@@ -1526,7 +1526,7 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
                                energy_lds(c->two_d, mixed), c->stream, ea);
             HIPCHK(c, hipGetLastError());
             hipLaunchKernelGGL(reduce_partials_kernel, dim3((kNPart + kReduceCols - 1) / kReduceCols, q1 - q0),
-                               dim3(256), 0, c->stream, part, nblk, kNPart, c->d_result + out * kNPart,
+                               dim3(kReduceThreads), 0, c->stream, part, nblk, kNPart, c->d_result + out * kNPart,
                                q1 - q0 > 1 ? (const int *)list.seg : (const int *)nullptr);
             HIPCHK(c, hipGetLastError());
             return SN_OK;
@@ -1551,8 +1551,8 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
         hipLaunchKernelGGL(energy_grad_kernel, dim3(nblk), dim3(256), 0, c->stream, c->d_lat, c->d_reps, q,
                            c->d_offs, c->noff, g, part);
         HIPCHK(c, hipGetLastError());
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3((kNPart + kReduceCols - 1) / kReduceCols), dim3(256), 0,
-                           c->stream, part, nblk, kNPart, c->d_result + (all ? q * kNPart : 0),
+        hipLaunchKernelGGL(reduce_partials_kernel, dim3((kNPart + kReduceCols - 1) / kReduceCols),
+                           dim3(kReduceThreads), 0, c->stream, part, nblk, kNPart, c->d_result + (all ? q * kNPart : 0),
                            (const int *)nullptr);
         HIPCHK(c, hipGetLastError());
     }
