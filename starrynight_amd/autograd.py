@@ -77,18 +77,21 @@ class EnergyModel:
 class _LatticeEnergy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, p, lengths, J, E, s, model):
-        En = E.detach().to("cpu", torch.float64).numpy()
+        # the three parameter inputs in one transfer, the six scalar results in another
+        par = torch.cat([J.detach().reshape(1), E.detach().reshape(3), s.detach().reshape(1)])
+        par = par.to("cpu", torch.float64).numpy()
+        J, En, s = float(par[0]), par[1:4], float(par[4])
         if p.is_cuda:
             e, g, dparams = model.evaluate_device(p.detach().contiguous(),
-                                                  lengths.detach().to(p.device, torch.float64),
-                                                  float(J), En, float(s))
+                                                  lengths.detach().to(p.device, torch.float64), J, En, s)
         else:
             pn = p.detach().to("cpu", torch.float64).numpy()
             ln = lengths.detach().to("cpu", torch.float64).numpy()
-            e, g, dparams = model.evaluate(pn, ln, float(J), En, float(s))
+            e, g, dparams = model.evaluate(pn, ln, J, En, s)
             g = torch.from_numpy(g)
-        ctx.save_for_backward(g.to(p.device), torch.from_numpy(dparams).to(p.device))
-        return torch.tensor(e, dtype=torch.float64, device=p.device)
+        res = torch.from_numpy(np.append(dparams, e)).to(p.device)
+        ctx.save_for_backward(g.to(p.device), res[:5])
+        return res[5].clone()
 
     @staticmethod
     def backward(ctx, gout):

@@ -383,6 +383,41 @@ __global__ __launch_bounds__(256) void lattice_scan_kernel(const double4 *lat, l
     if (tid < 3) partials[(long long)blockIdx.x * 3 + tid] = red[tid][0];
 }
 
+// Second pass of a lattice written from device memory: every workgroup sums
+// up the scan's partials, and copies its share if nothing was non-finite; the
+// first also reports {count, min, max} to `verdict` (pinned host memory).
+__global__ __launch_bounds__(256) void lattice_take_kernel(const double4 *src, double4 *dst, long long N,
+                                                           const double *partials, int nblk, double *verdict)
+{
+    __shared__ double red[3][4];
+    const int tid = threadIdx.x;
+    double bad = 0.0, lo = INFINITY, hi = -INFINITY;
+    for (int b = tid; b < nblk; b += 256) {
+        bad += partials[3 * b];
+        lo = fmin(lo, partials[3 * b + 1]);
+        hi = fmax(hi, partials[3 * b + 2]);
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        bad += __shfl_xor(bad, o, 64);
+        lo = fmin(lo, __shfl_xor(lo, o, 64));
+        hi = fmax(hi, __shfl_xor(hi, o, 64));
+    }
+    if ((tid & 63) == 0) { red[0][tid >> 6] = bad; red[1][tid >> 6] = lo; red[2][tid >> 6] = hi; }
+    __syncthreads();
+    bad = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    if (blockIdx.x == 0 && tid == 0) {
+        verdict[0] = bad;
+        verdict[1] = fmin(fmin(red[1][0], red[1][1]), fmin(red[1][2], red[1][3]));
+        verdict[2] = fmax(fmax(red[2][0], red[2][1]), fmax(red[2][2], red[2][3]));
+    }
+    if (bad > 0.0) return;   // uniform
+    for (long long s = (long long)blockIdx.x * 256 + tid; s < N; s += (long long)gridDim.x * 256) dst[s] = src[s];
+}
+
+// A replica's record, passed as an argument: in stream order, no copy to wait for.
+__global__ void put_rep_kernel(RepDev *dst, RepDev rep) { *dst = rep; }
+
 // Random initial lattice on the device: unit dipole from the counter RNG
 // (stream tag 0xFFFFFFFF in the sweep slot) and a length drawn from the
 // species table (cumulative prevalence walk, as solid_solution does).

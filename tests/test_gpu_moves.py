@@ -23,7 +23,7 @@ def test_moves_of_any_count(sn, oracle, dims, rc):
     o = oracle_model(oracle, rp)
     with sn.StarryNight(rp) as ctx:
         ctx.set_lattice(lat)
-        for n in (1, 16, 17, 33000):
+        for n in (1, 16, 17, 1024, 1025, 33000):
             sites = rng.integers(0, rp.N, n).astype(np.int32)
             props = rand_lattice(n, rng, mixed=False)[:, :3].copy()
             got = ctx.site_energy_batch(sites, props)
