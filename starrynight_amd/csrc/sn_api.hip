@@ -310,9 +310,10 @@ static T *stage_ptr(sn_ctx *c, size_t offset)
 
 // Lists of at most this many moves are read, and their energies written, by
 // the kernel itself in pinned host memory (5 doubles a move: proposal, energy,
-// site) instead of three copies: one move 34.7 -> 21.4 us.  Longer lists keep
-// the copies, which read host memory in larger pieces.
-constexpr int kPinnedMoves = 1024, kMoveDoubles = 5;
+// site) instead of three copies: one move 34.7 -> 21.4 us, 8000 of a 30^3
+// lattice 62 -> 36 us.  The bound is what a context may pin (640 KB); longer
+// lists keep the copies.
+constexpr int kPinnedMoves = 16384, kMoveDoubles = 5;
 
 // HIP events destroyed when the list goes out of scope (every return path).
 struct EventList {
@@ -1162,10 +1163,16 @@ int sn_site_energy_batch_device(sn_ctx *c, int32_t r, int64_t n, const int32_t *
     if (n < 0) return fail(c, SN_ERR_INVALID, "negative count");
     if (n == 0) return SN_OK;
     if (!site || !prop || !dE) return fail(c, SN_ERR_INVALID, "null buffer");
-    const long long per_block = kMoveThreads / kMoveLanes;
+    const int lanes = move_lanes(c->noff);
+    const long long per_block = kMoveThreads / lanes;
     const unsigned nb = (unsigned)std::min<long long>((n + per_block - 1) / per_block, kMoveBlocks);
-    hipLaunchKernelGGL(site_energy_batch_kernel, dim3(nb), dim3(kMoveThreads), move_lds(c->noff), c->stream, c->d_lat,
-                       c->d_reps, r, c->d_offs, c->noff, (long long)n, site, prop, dE);
+    const auto kernel = lanes == 1   ? site_energy_batch_kernel<1>
+                        : lanes == 2 ? site_energy_batch_kernel<2>
+                        : lanes == 4 ? site_energy_batch_kernel<4>
+                        : lanes == 8 ? site_energy_batch_kernel<8>
+                                     : site_energy_batch_kernel<16>;
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(kMoveThreads), move_lds(c->noff), c->stream, c->d_lat, c->d_reps, r,
+                       c->d_offs, c->noff, (long long)n, site, prop, dE);
     HIPCHK(c, hipGetLastError());
     return SN_OK;
 }

@@ -38,19 +38,37 @@ __device__ __forceinline__ void site_field(const double4 *lat, const RepDev &rep
     }
 }
 
-// Energy differences of proposed moves.  16 lanes share a move: lanes next to
+// Energy differences of proposed moves.  G lanes share a move: lanes next to
 // each other read offsets next to each other, mostly one run along z, so a
 // gather touches a third of the cache lines that 64 moves a wave did, and a
 // single move has its neighbours in flight together.  The offset table is in
 // LDS, padded with zero weights to a whole number of rounds; groups take moves
 // in turn until none is left.  100000 moves of a 64^3 lattice at cut-off 3:
 // 53 us (99 us with a move per lane), one move 2.8 us (10 us); bound by the
-// gathers' cache lines.
-constexpr int kMoveLanes = 16, kMoveThreads = 256;
+// gathers' cache lines.  G is the power of two, at most 16, that leaves about
+// four rounds, whose gathers are in flight together: fewer lanes for short
+// tables, since a move's own work (site, proposal, result) is done by each of
+// its lanes.  A call of 200000 moves: 64^3, cut-off 1, 354 us with 2 lanes, 367
+// with 16; 2D, cut-off 2, 358 us with 4, 369 with 16 (mostly copies).
+constexpr int kMoveThreads = 256;
 constexpr int kMoveBlocks = 2048;   // eight workgroups a CU
 
-__host__ __device__ inline int move_table(int noff) { return (noff + kMoveLanes - 1) / kMoveLanes * kMoveLanes; }
-inline size_t move_lds(int noff) { return (size_t)move_table(noff) * (sizeof(double2) + sizeof(int2)); }
+__host__ __device__ inline int move_lanes(int noff)
+{
+    int G = 1;
+    while (G < 16 && 4 * G < noff) G *= 2;
+    return G;
+}
+__host__ __device__ inline int move_rounds(int noff, int G)
+{
+    const int rounds = (noff + G - 1) / G;
+    return rounds < 4 ? 4 : rounds;
+}
+inline size_t move_lds(int noff)
+{
+    const int G = move_lanes(noff);
+    return (size_t)move_rounds(noff, G) * G * (sizeof(double2) + sizeof(int2));
+}
 
 // q = s / d and the remainder, for 0 <= s < 2^31: id = 1 / d is within an ulp,
 // so the quotient is at most one off.
@@ -63,15 +81,16 @@ __device__ __forceinline__ int divide(int s, int d, double id, int &rest)
     return q;
 }
 
+template <int G>
 __global__ __launch_bounds__(kMoveThreads) void site_energy_batch_kernel(
     const double4 *__restrict__ lat, const RepDev *__restrict__ reps, int replica,
     const PairDev *__restrict__ offs, int noff, long long n, const int *__restrict__ site,
     const double *__restrict__ prop, double *__restrict__ dE)
 {
     extern __shared__ double2 s_w[];   // w, 3 w / |r|^2
-    const int rounds = move_table(noff) / kMoveLanes;
-    int2 *const s_d = (int2 *)(s_w + rounds * kMoveLanes);   // dx, dy; dz, nearest neighbour
-    for (int i = threadIdx.x; i < rounds * kMoveLanes; i += kMoveThreads) {
+    const int rounds = move_rounds(noff, G);
+    int2 *const s_d = (int2 *)(s_w + rounds * G);   // dx, dy; dz, nearest neighbour
+    for (int i = threadIdx.x; i < rounds * G; i += kMoveThreads) {
         double2 w = make_double2(0.0, 0.0);
         int2 d = make_int2(0, 0);
         if (i < noff) {
@@ -87,9 +106,9 @@ __global__ __launch_bounds__(kMoveThreads) void site_energy_batch_kernel(
     const double4 *L = lat + rep.base;
     const long long N = (long long)rep.X * rep.Y * rep.Z;
     const double iY = 1.0 / rep.Y, iZ = 1.0 / rep.Z;
-    const int lane = threadIdx.x % kMoveLanes;
-    const long long step = (long long)gridDim.x * (kMoveThreads / kMoveLanes);
-    for (long long k = (long long)blockIdx.x * (kMoveThreads / kMoveLanes) + threadIdx.x / kMoveLanes; k < n; k += step) {
+    const int lane = threadIdx.x % G;
+    const long long step = (long long)gridDim.x * (kMoveThreads / G);
+    for (long long k = (long long)blockIdx.x * (kMoveThreads / G) + threadIdx.x / G; k < n; k += step) {
         const int s = site[k];
         const double px = prop[3 * k], py = prop[3 * k + 1], pz = prop[3 * k + 2];
         // an index outside the replica reads nothing and yields NaN
@@ -122,21 +141,21 @@ __global__ __launch_bounds__(kMoveThreads) void site_energy_batch_kernel(
             int2 d[4];
             double4 q[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) q[j] = offset((t + j) * kMoveLanes + lane, d[j]);
+            for (int j = 0; j < 4; j++) q[j] = offset((t + j) * G + lane, d[j]);
 #pragma unroll
-            for (int j = 0; j < 4; j++) add((t + j) * kMoveLanes + lane, d[j], q[j]);
+            for (int j = 0; j < 4; j++) add((t + j) * G + lane, d[j], q[j]);
         }
         for (; t < rounds; t++) {
             int2 d;
-            const double4 q = offset(t * kMoveLanes + lane, d);
-            add(t * kMoveLanes + lane, d, q);
+            const double4 q = offset(t * G + lane, d);
+            add(t * G + lane, d, q);
         }
-        f.hx = group_sum_dpp<kMoveLanes>(f.hx);
-        f.hy = group_sum_dpp<kMoveLanes>(f.hy);
-        f.hz = group_sum_dpp<kMoveLanes>(f.hz);
-        f.gx = group_sum_dpp<kMoveLanes>(f.gx);
-        f.gy = group_sum_dpp<kMoveLanes>(f.gy);
-        f.gz = group_sum_dpp<kMoveLanes>(f.gz);
+        f.hx = group_sum_dpp<G>(f.hx);
+        f.hy = group_sum_dpp<G>(f.hy);
+        f.hz = group_sum_dpp<G>(f.hz);
+        f.gx = group_sum_dpp<G>(f.gx);
+        f.gy = group_sum_dpp<G>(f.gy);
+        f.gz = group_sum_dpp<G>(f.gz);
         double e = o.w * (dx * f.hx + dy * f.hy + dz * f.hz) - rep.J * (dx * f.gx + dy * f.gy + dz * f.gz) +
                    (dx * rep.E[0] + dy * rep.E[1] + dz * rep.E[2]);
         if (rep.K > 0.0) e += -rep.K * (fabs(px) - fabs(o.x) + fabs(py) - fabs(o.y));

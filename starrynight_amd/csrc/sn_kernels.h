@@ -87,7 +87,7 @@ __device__ __forceinline__ double pair_sum_f64(double v)
 template <int G>
 __device__ __forceinline__ double group_sum_dpp(double v)
 {
-    static_assert(G == 2 || G == 4 || G == 8 || G == 16 || G == 32 || G == 64, "G is a power of two <= 64");
+    static_assert(G == 1 || G == 2 || G == 4 || G == 8 || G == 16 || G == 32 || G == 64, "G is a power of two <= 64");
     if (G >= 64) v = pair_sum_f64<32>(v);
     if (G >= 32) v = pair_sum_f64<16>(v);
     if (G >= 16) v += dpp_f64<0x140>(v);
