@@ -100,8 +100,8 @@ struct sn_ctx {
     // reductions (at least 256), then the moves of short lists
     double *h_result = nullptr, *d_result = nullptr;
     size_t moves_off = 0;                // doubles before the moves
-    std::vector<int> rep_tiles;          // tiles per replica
-    bool energy_tiled = false;           // energy / gradient through tile_energy_kernel
+    std::vector<int> scratch_rows;       // rows of the fixed scratch a replica counts for (its tiles; empty: no tiling)
+    bool energy_rows = false;            // energy / gradient through energy_kernel (cut-offs 1..5)
     // whole-lattice sweeps of small replicas (kernel 3): one workgroup per replica
     bool torus = false;
     Sublattice torus_lat{};
@@ -977,18 +977,19 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
         else if (ts != SN_ERR_UNSUPPORTED) return ts;
         else c->err = keep;
     }
-    if (!tiles_ok) return SN_OK;
-    // (cut-offs whose tiles the energy kernel was first built on)
-    if (pick_energy(c->rc, c->two_d, false, false) && (size_t)4 * field_region_doubles(c) * sizeof(double) <= 150 * 1024) {
-        c->rep_tiles.assign(c->R, 0);
-        for (const Tile &t : c->sched.tiles) c->rep_tiles[t.replica]++;
+    if (pick_energy(c->rc, c->two_d, false, false)) {
+        if (tiles_ok && (size_t)4 * field_region_doubles(c) * sizeof(double) <= 150 * 1024) {
+            c->scratch_rows.assign(c->R, 0);
+            for (const Tile &t : c->sched.tiles) c->scratch_rows[t.replica]++;
+        }
         if ((st = energy_list(c, true, c->energy_all)) || (st = energy_list(c, false, c->energy_each))) return st;
         for (int m = 0; m < 4; m++)
             HIPCHK(c, hipFuncSetAttribute((const void *)pick_energy(c->rc, c->two_d, m & 1, m & 2),
                                           hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)energy_lds(c->two_d, m & 1)));
-        c->energy_tiled = true;
+        c->energy_rows = true;
     }
+    if (!tiles_ok) return SN_OK;
     for (int m = 0; m < 2; m++) {
         const void *f = c->use_field
                             ? (const void *)pick_field(c->rc, c->two_d, m == 1)
@@ -1513,9 +1514,10 @@ int sn_set_sweep_index(sn_ctx *c, int32_t r, uint64_t index)
 }
 
 // Energy parts and parameter derivatives (kNPart sums per replica into
-// d_result) and the gradient into dg when non-null.  Lattices with a sweep
-// schedule and DipoleCutOff <= 5 take the tiled kernel (one workgroup per
-// tile, LDS-staged stencil), the others the per-site gather kernel.
+// d_result) and the gradient into dg when non-null.  DipoleCutOff <= 5 takes
+// energy_kernel, which needs no tiling (lattices without one took the per-site
+// kernel, a launch per replica: 16 replicas of 16^3 at cut-off 5 2236 us, now
+// 48 us); beyond 5 the per-site gather kernel.
 // r >= 0: replica r alone, dg holds its N x 3 rows.  r < 0: every replica,
 // dg holds all sites' rows in lattice order (replica r from row base_r), and
 // replica r's sums land at d_result + r * kNPart.
@@ -1540,10 +1542,13 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
         return e;
     };
     double *part = nullptr;
-    if (c->energy_tiled) {
-        int tiles = 0;
-        for (int q = all ? 0 : r; q < (all ? c->R : r + 1); q++) tiles += c->rep_tiles[q];
-        if (fixed_partials && (st = partials((size_t)tiles * kNPart, &part))) return st;   // (a row per tile)
+    if (c->energy_rows) {
+        if (fixed_partials) {   // a row per tile, or per 256 sites of the largest replica without tiles
+            long long rows = 0;
+            for (int q = all ? 0 : r; q < (all ? c->R : r + 1); q++)
+                rows = c->scratch_rows.empty() ? std::max(rows, (c->reps[q].N + 255) / 256) : rows + c->scratch_rows[q];
+            if ((st = partials((size_t)rows * kNPart, &part))) return st;
+        }
         // one launch over replicas q0..q1-1, whose sums go to d_result + out * kNPart
         auto launch = [&](const EnergyList &list, int q0, int q1, bool mixed, double *g, int out) -> int {
             const int nblk = list.off[q1] - list.off[q0];
@@ -1562,7 +1567,7 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
         };
         if (!all) return launch(c->energy_each, r, r + 1, c->reps[r].mixed != 0, dg, 0);
         // one launch (the mixed-length variant serves uniform replicas too),
-        // or, where the fixed scratch holds a row per tile but not one per
+        // or, where the fixed scratch does not hold a row per
         // workgroup, a launch per replica: they use it in stream order
         if (!fixed_partials || (size_t)c->energy_all.off[c->R] * kNPart <= fixed_cap)
             return launch(c->energy_all, 0, c->R, any_mixed(c), dg, 0);

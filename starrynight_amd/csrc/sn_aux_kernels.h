@@ -1,7 +1,8 @@
-// sn_aux_kernels.h -- gather kernels beside the tile sweep (gfx950, FP64):
+// sn_aux_kernels.h -- kernels beside the tile sweep (gfx950, FP64):
 // sweep-counter bump, the site_energy batch, sequential replay, energy /
-// adjoint, reductions, moment and the random initial lattice.  Included by
-// sn_api.hip only (non-template kernels: one definition).
+// adjoint beyond cut-off 5, reductions, moment, device lattices, the random
+// initial lattice and the recombination sums.  Included by sn_api.hip only
+// (non-template kernels: one definition).
 #pragma once
 #include "sn_kernels.h"
 
@@ -12,8 +13,8 @@ __global__ void bump_sweep_kernel(unsigned *sweep_ctr, int R, unsigned n)
     if (r < R) sweep_ctr[r] += n;
 }
 
-// Local field pieces of one site by direct gathers from HBM (used by the
-// site_energy batch, the replay and the energy / adjoint kernels).
+// Local field pieces of one site (the site_energy batch), and by direct
+// gathers from HBM (energy / adjoint beyond cut-off 5).
 struct FieldOut {
     double hx, hy, hz;  // sum_r L_j (p_j - 3 n (n.p_j)) / d^3
     double gx, gy, gz;  // sum_{|r|=1} p_j
@@ -250,7 +251,7 @@ __global__ __launch_bounds__(256) void replay_kernel(double4 *lat, const RepDev 
     if (tid == 0) { stats[0] = mism; stats[1] = ties; stats[2] = nacc; stats[3] = nrej; }
 }
 
-// Energy and adjoint: one site per lane; per-site gradient dE/dp_i and
+// Energy and adjoint at cut-offs beyond energy_kernel's: one site per lane; per-site gradient dE/dp_i and
 // per-workgroup partial sums of
 //   {E_dd, E_cage, E_field, E_K, dE/dJ, dE/dEx, dE/dEy, dE/dEz, dE/ds, dE/dK}.
 constexpr int kNPart = 10;

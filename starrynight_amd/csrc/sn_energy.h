@@ -146,7 +146,8 @@ __global__ __launch_bounds__(kEnergyThreads) void energy_kernel(EnergyArgs ea)
     double4 v[2][NL];   // planes on their way, by parity
     auto load = [&](int x0, auto ic) __attribute__((always_inline)) {
         constexpr int I = decltype(ic)::value;
-        const double4 *plane = lat + (long long)wrap_once(x0 - RC + I, rep.X) * rep.Y * Z;
+        // (twice: the last step of a short axis reaches beyond its second copy)
+        const double4 *plane = lat + (long long)wrap_once(wrap_once(x0 - RC + I, rep.X), rep.X) * rep.Y * Z;
 #pragma unroll
         for (int j = 0; j < NL; j++) v[I & 1][j] = plane[at_plane[j]];
     };

@@ -49,9 +49,11 @@ def test_stencil_tiles(sn, oracle, dims):
 
 # rows held whole or cut (Z = 180: halo inside the lattice), rows and x left
 # over by the workgroups, workgroups of several steps along x, one and two x a
-# step, plane (2D) lattices of more rows than lanes
+# step, plane (2D) lattices of more rows than lanes, an axis of two sites,
+# lattices without a tiling
 ENERGY = [((8, 7, 6), 3), ((7, 30, 5), 2), ((9, 12, 180), 4), ((10, 9, 70), 1), ((33, 20, 16), 5), ((16, 600, 1), 3),
-          ((300, 10, 1), 5), ((64, 64, 64), 3)]
+          ((300, 10, 1), 5), ((64, 64, 64), 3),
+          ((2, 40, 5), 1), ((6, 7, 8), 5), ((6, 9, 1), 5)]
 
 
 @pytest.mark.parametrize("mixed", [False, True])
