@@ -121,6 +121,7 @@ int sn_reference_initial_lattice(int32_t X, int32_t Y, int32_t Z, const char *in
 
 /* Change T, Efield and CageStrain of replica r between sweeps (temperature
  * schedules, field ramps) without rebuilding the schedule or the graph.
+ * Takes effect in the order of the context's stream, without waiting for it.
  * Replaces assignments to the globals beta / Efield / CageStrain
  * (src/starrynight-main.c:215, 239). */
 int sn_set_params(sn_ctx *ctx, int32_t replica, double temperature, const double efield[3],
@@ -192,7 +193,7 @@ int sn_gradient(sn_ctx *ctx, int32_t replica, double *grad_p, double dparams[6],
  * NULL) written in place: no host copy of the N x 3 field.  Returns after
  * grad_dev is written. */
 int sn_gradient_device(sn_ctx *ctx, int32_t replica, void *grad_dev, double dparams[6], double *energy);
-/* Every replica's adjoint in one pass (one launch over all replicas' tiles).
+/* Every replica's adjoint in one pass (one launch over all replicas).
  * grad_dev (device, may be NULL) holds 3 doubles per site of all replicas in
  * lattice order: replica r's rows start after the sites of replicas 0..r-1.
  * dparams (double[R][6]) and energy (double[R]) may be NULL. */
