@@ -227,12 +227,4 @@ __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n)
     return xcd * each + min(xcd, rest) + b / 8;
 }
 
-template <int G>
-__device__ __forceinline__ double group_sum(double v)
-{
-#pragma unroll
-    for (int o = 1; o < G; o <<= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
 }  // namespace sn
