@@ -205,6 +205,7 @@ static int ensure_partials(sn_ctx *c, size_t n)
     if (n <= c->partial_cap) return SN_OK;
     if (c->d_partials) (void)hipFree(c->d_partials);
     c->d_partials = nullptr;
+    c->partial_cap = 0;   // (a failed allocation leaves no buffer)
     HIPCHK(c, hipMalloc((void **)&c->d_partials, n * sizeof(double)));
     c->partial_cap = n;
     return SN_OK;

@@ -1,0 +1,125 @@
+/* A stand-in for the HIP runtime on a machine without a GPU: device memory is
+ * host memory, kernels do not run, and what the library asks of the runtime is
+ * written down (launches, bytes copied to the device).  Allocations beyond a
+ * limit fail, and a stream can be said to be under capture. */
+#include <stdint.h>
+#include <stdlib.h>
+#include <string.h>
+
+typedef struct { uint32_t x, y, z; } dim3_t;
+enum { OK = 0, OUT_OF_MEMORY = 2, INVALID_VALUE = 1, H2D = 1 };
+
+size_t si_malloc_limit = SIZE_MAX; /* larger device allocations fail */
+size_t si_uploaded;                /* bytes copied host to device */
+int si_copy_fails;                 /* synchronous copies fail */
+int si_capturing;                  /* every stream is under capture */
+int si_last_error;                 /* what hipGetLastError returns */
+
+/* ---- launches ---- */
+enum { MAX_KERNELS = 4096, KEEP = 64 };
+static struct { const void *host; const char *name; } kernels[MAX_KERNELS];
+static int n_kernels;
+typedef struct { char name[256]; uint32_t grid[3], block[3]; size_t lds; unsigned char arg[128]; } launch_t;
+launch_t si_launch[KEEP]; /* the last KEEP launches, at index number % KEEP */
+long si_launches;
+
+static const char *kernel_name(const void *host)
+{
+    for (int i = 0; i < n_kernels; i++)
+        if (kernels[i].host == host) return kernels[i].name;
+    return "?";
+}
+
+int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t lds, void *stream)
+{
+    (void)stream;
+    launch_t *l = &si_launch[si_launches++ % KEEP];
+    memset(l, 0, sizeof *l);
+    strncpy(l->name, kernel_name(f), sizeof l->name - 1);
+    l->grid[0] = g.x; l->grid[1] = g.y; l->grid[2] = g.z;
+    l->block[0] = b.x; l->block[1] = b.y; l->block[2] = b.z;
+    l->lds = lds;
+    /* the argument a test looks at: the partial sums, the parameter record */
+    if (strstr(l->name, "moment_kernel")) memcpy(l->arg, args[3], sizeof(void *));
+    if (strstr(l->name, "put_rep_kernel")) memcpy(l->arg, args[1], 96);
+    return OK;
+}
+
+static dim3_t cfg_grid, cfg_block;
+static size_t cfg_lds;
+static void *cfg_stream;
+int __hipPushCallConfiguration(dim3_t g, dim3_t b, size_t lds, void *stream)
+{
+    cfg_grid = g; cfg_block = b; cfg_lds = lds; cfg_stream = stream;
+    return OK;
+}
+int __hipPopCallConfiguration(dim3_t *g, dim3_t *b, size_t *lds, void **stream)
+{
+    *g = cfg_grid; *b = cfg_block; *lds = cfg_lds; *stream = cfg_stream;
+    return OK;
+}
+static void *module;
+void **__hipRegisterFatBinary(const void *data) { (void)data; return &module; }
+void __hipUnregisterFatBinary(void **m) { (void)m; }
+void __hipRegisterFunction(void **m, const void *host, char *device, const char *name, unsigned limit, void *t, void *b,
+                           void *bd, void *gd, int *w)
+{
+    (void)m; (void)device; (void)limit; (void)t; (void)b; (void)bd; (void)gd; (void)w;
+    if (n_kernels < MAX_KERNELS) { kernels[n_kernels].host = host; kernels[n_kernels++].name = name; }
+}
+void __hipRegisterVar(void **m, void *var, char *h, char *d, int ext, size_t size, int constant, int global)
+{
+    (void)m; (void)var; (void)h; (void)d; (void)ext; (void)size; (void)constant; (void)global;
+}
+
+/* ---- memory ---- */
+int hipMalloc(void **p, size_t n)
+{
+    if (n > si_malloc_limit) return OUT_OF_MEMORY;
+    *p = calloc(n ? n : 1, 1);
+    return *p ? OK : OUT_OF_MEMORY;
+}
+int hipFree(void *p) { free(p); return OK; }
+int hipHostMalloc(void **p, size_t n, unsigned flags) { (void)flags; *p = calloc(n ? n : 1, 1); return *p ? OK : OUT_OF_MEMORY; }
+int hipHostFree(void *p) { free(p); return OK; }
+int hipHostGetDevicePointer(void **d, void *h, unsigned flags) { (void)flags; *d = h; return OK; }
+static int copy(void *d, const void *s, size_t n, int kind)
+{
+    if (kind == H2D) si_uploaded += n;
+    memcpy(d, s, n);
+    return OK;
+}
+int hipMemcpy(void *d, const void *s, size_t n, int kind) { return si_copy_fails ? INVALID_VALUE : copy(d, s, n, kind); }
+int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *stream) { (void)stream; return copy(d, s, n, kind); }
+int hipMemset(void *d, int v, size_t n) { memset(d, v, n); return OK; }
+int hipGetSymbolAddress(void **p, const void *symbol)
+{
+    static void *scratch;
+    (void)symbol;
+    if (!scratch) scratch = calloc(1 << 21, 1);
+    *p = scratch;
+    return scratch ? OK : OUT_OF_MEMORY;
+}
+
+/* ---- device, streams, events, graphs ---- */
+static int handle;
+int hipGetDevice(int *d) { *d = 0; return OK; }
+int hipDeviceGetAttribute(int *v, int attribute, int device) { (void)attribute; (void)device; *v = 256; return OK; }
+int hipGetDevicePropertiesR0600(void *p, int device) { (void)p; (void)device; return INVALID_VALUE; }
+int hipFuncSetAttribute(const void *f, int attribute, int value) { (void)f; (void)attribute; (void)value; return OK; }
+const char *hipGetErrorString(int e) { return e == OUT_OF_MEMORY ? "out of memory" : "error"; }
+int hipGetLastError(void) { int e = si_last_error; si_last_error = 0; return e; }
+int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &handle; return OK; }
+int hipStreamDestroy(void *s) { (void)s; return OK; }
+int hipStreamSynchronize(void *s) { (void)s; return OK; }
+int hipStreamIsCapturing(void *s, int *status) { (void)s; *status = si_capturing; return OK; }
+int hipStreamBeginCapture(void *s, int mode) { (void)s; (void)mode; return OK; }
+int hipStreamEndCapture(void *s, void **graph) { (void)s; *graph = &handle; return OK; }
+int hipGraphInstantiate(void **e, void *g, void *n, char *log, size_t size) { (void)g; (void)n; (void)log; (void)size; *e = &handle; return OK; }
+int hipGraphLaunch(void *e, void *s) { (void)e; (void)s; return OK; }
+int hipGraphExecDestroy(void *e) { (void)e; return OK; }
+int hipGraphDestroy(void *g) { (void)g; return OK; }
+int hipEventCreate(void **e) { *e = &handle; return OK; }
+int hipEventDestroy(void *e) { (void)e; return OK; }
+int hipEventRecord(void *e, void *s) { (void)e; (void)s; return OK; }
+int hipEventElapsedTime(float *ms, void *a, void *b) { (void)a; (void)b; *ms = 0.0f; return OK; }

@@ -1,0 +1,72 @@
+"""The library's host side on a stand-in HIP runtime (no GPU): what it does when
+the runtime refuses something, and what it asks the runtime for.
+
+tests/hip_stand_in.c takes the place of the HIP runtime in a process of its
+own; device memory is host memory there and kernels do not run.  Each test
+runs a short script against the C ABI and reads what it prints.
+"""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = r"""
+import ctypes as C, struct, sys
+si = C.CDLL(sys.argv[1], C.RTLD_GLOBAL)       # its symbols come before the runtime's
+from starrynight_amd._lib import LIB_PATH, Params, Tuning
+L = C.CDLL(LIB_PATH)
+vp = C.c_void_p
+L.sn_last_error.restype = C.c_char_p
+class Launch(C.Structure):
+    _fields_ = [("name", C.c_char * 256), ("grid", C.c_uint32 * 3), ("block", C.c_uint32 * 3), ("lds", C.c_size_t),
+                ("arg", C.c_ubyte * 128)]
+limit, uploaded = C.c_size_t.in_dll(si, "si_malloc_limit"), C.c_size_t.in_dll(si, "si_uploaded")
+capturing, copy_fails = C.c_int.in_dll(si, "si_capturing"), C.c_int.in_dll(si, "si_copy_fails")
+def launches():
+    n, ring = C.c_long.in_dll(si, "si_launches").value, (Launch * 64).in_dll(si, "si_launch")
+    return [ring[k % 64] for k in range(max(0, n - 64), n)]
+def last(name):
+    return [l for l in launches() if name.encode() in l.name][-1]
+def create(boxes, rc=3, T=300.0, kernel=0):
+    ps = (Params * len(boxes))()
+    for p, (p.X, p.Y, p.Z) in zip(ps, boxes):
+        p.dipole_cutoff, p.cage_strain, p.temperature = rc, 1.0, T
+    t, h = Tuning(kernel=kernel), vp()
+    status = L.sn_create(ps, len(boxes), C.byref(t), C.byref(h))
+    return status, h
+def context(*args, **kw):
+    status, h = create(*args, **kw)
+    assert status == 0, L.sn_last_error(h)
+    return h
+D = C.c_double
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = tmp_path_factory.mktemp("stand_in") / "hip_stand_in.so"
+    subprocess.check_call(["gcc", "-O1", "-Wall", "-shared", "-fPIC", "-o", str(so),
+                           os.path.join(ROOT, "tests", "hip_stand_in.c")])
+
+    def script(body):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + body, str(so)], cwd=ROOT, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr
+        return r.stdout.split()
+    return script
+
+
+def test_partial_sums_are_never_a_null_buffer(run):
+    """A larger buffer that cannot be had is an error, and so is not forgotten:
+    the next call that needs no more than the old size gets a buffer again."""
+    out = run(r"""
+h = context([(64, 64, 64), (12, 12, 12)])
+fe, afe, count, M = (D * 81)(), (D * 81)(), (C.c_int64 * 81)(), (D * 3)()
+print(L.sn_moment(h, 0, M))                      # a first buffer
+limit.value = 100000
+print(L.sn_radial_order(h, 0, fe, afe, count))   # needs a larger one
+print(L.sn_moment(h, 1, M), struct.unpack("<Q", bytes(last("moment_kernel").arg[:8]))[0] != 0)
+""")
+    assert out == ["0", "2", "0", "True"]
