@@ -200,6 +200,20 @@ static int upload(sn_ctx *c, T **dst, const std::vector<T> &v)
     return SN_OK;
 }
 
+// A table built on first use: kept only when it is on the device.
+static int upload_table(sn_ctx *c, void **table, const void *src, size_t bytes)
+{
+    void *dev = nullptr;
+    HIPCHK(c, hipMalloc(&dev, bytes));
+    const hipError_t e = hipMemcpy(dev, src, bytes, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        (void)hipFree(dev);
+        return fail(c, SN_ERR_HIP, std::string("copy of a table: ") + hipGetErrorString(e));
+    }
+    *table = dev;
+    return SN_OK;
+}
+
 static int ensure_partials(sn_ctx *c, size_t n)
 {
     if (n <= c->partial_cap) return SN_OK;
@@ -1738,13 +1752,9 @@ static int ensure_radial(sn_ctx *c)
     std::memcpy(table.data(), cols.data(), at_start);
     std::memcpy(table.data() + at_start, start.data(), start.size() * sizeof(int));
     std::memcpy(table.data() + at_entries, entries.data(), entries.size() * sizeof(unsigned short));
-    char *dev = nullptr;
-    HIPCHK(c, hipMalloc((void **)&dev, table.size()));
-    c->d_radial = dev;
     c->radial_start = at_start;
     c->radial_entries = at_entries;
-    HIPCHK(c, hipMemcpy(dev, table.data(), table.size(), hipMemcpyHostToDevice));
-    return SN_OK;
+    return upload_table(c, &c->d_radial, table.data(), table.size());
 }
 
 // Workgroups of 4 rows x tz sites, each over a range of x.  A workgroup stages
@@ -1830,11 +1840,7 @@ static int ensure_stencil(sn_ctx *c, int kind)
             }
     HIPCHK(c, hipFuncSetAttribute((const void *)pick_stencil(kind), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)stencil_lds(R)));
-    double *dev = nullptr;
-    HIPCHK(c, hipMalloc((void **)&dev, weights.size() * sizeof(double)));
-    c->d_stencil[kind] = dev;
-    HIPCHK(c, hipMemcpy(dev, weights.data(), weights.size() * sizeof(double), hipMemcpyHostToDevice));
-    return SN_OK;
+    return upload_table(c, (void **)&c->d_stencil[kind], weights.data(), weights.size() * sizeof(double));
 }
 
 // Launches the stencil of `kind` into d_obs (width values per site).

@@ -70,3 +70,20 @@ print(L.sn_radial_order(h, 0, fe, afe, count))   # needs a larger one
 print(L.sn_moment(h, 1, M), struct.unpack("<Q", bytes(last("moment_kernel").arg[:8]))[0] != 0)
 """)
     assert out == ["0", "2", "0", "True"]
+
+
+@pytest.mark.parametrize("call", ["L.sn_radial_order(h, 0, fe, afe, count)", "L.sn_dipole_potential(h, 0, pot)"])
+def test_observable_tables_are_kept_only_when_filled(run, call):
+    """A table whose copy to the device failed is made again on the next call."""
+    out = run(rf"""
+h = context([(12, 12, 12)])
+fe, afe, count, pot = (D * 81)(), (D * 81)(), (C.c_int64 * 81)(), (D * 1728)()
+copy_fails.value = 1
+print({call})
+copy_fails.value = 0
+before = uploaded.value
+print({call}, uploaded.value > before)
+before = uploaded.value
+print({call}, uploaded.value > before)           # kept from now on
+""")
+    assert out == ["2", "0", "True", "0", "False"]
