@@ -167,16 +167,27 @@ static RepDev make_repdev(const sn_params &p, const RepHost &h)
     return d;
 }
 
-// Replica r's parameters to the device, in stream order after what is queued.
-static int upload_rep(sn_ctx *c, int r)
+// Parameter records are not changed by a captured launch: each replay would set them again.
+static int check_not_capturing(sn_ctx *c)
 {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     HIPCHK(c, hipStreamIsCapturing(c->stream, &capture));
-    if (capture != hipStreamCaptureStatusNone)   // (a replay would set these parameters again)
+    if (capture != hipStreamCaptureStatusNone)
         return fail(c, SN_ERR_HIP, "parameters set while the context's stream is being captured");
-    hipLaunchKernelGGL(put_rep_kernel, dim3(1), dim3(1), 0, c->stream, c->d_reps + r,
-                       make_repdev(c->params[r], c->reps[r]));
+    return SN_OK;
+}
+
+// Replica r takes parameters p and lattice state h: to the device, in stream
+// order after what is queued, then into the context, which keeps what it had
+// if the launch was refused.
+static int set_rep(sn_ctx *c, int r, const sn_params &p, const RepHost &h)
+{
+    int st;
+    if ((st = check_not_capturing(c))) return st;
+    hipLaunchKernelGGL(put_rep_kernel, dim3(1), dim3(1), 0, c->stream, c->d_reps + r, make_repdev(p, h));
     HIPCHK(c, hipGetLastError());
+    c->params[r] = p;
+    c->reps[r] = h;
     return SN_OK;
 }
 
@@ -1055,7 +1066,7 @@ int sn_set_lattice(sn_ctx *c, int32_t r, const double *xyzl)
     int st = check_rep(c, r);
     if (st) return st;
     if (!xyzl) return fail(c, SN_ERR_INVALID, "null lattice buffer");
-    RepHost &h = c->reps[r];
+    RepHost h = c->reps[r];
     double L0 = xyzl[3];
     int mixed = 0;
     for (long long i = 0; i < h.N; i++) {
@@ -1068,7 +1079,7 @@ int sn_set_lattice(sn_ctx *c, int32_t r, const double *xyzl)
     HIPCHK(c, hipMemcpy(c->d_lat + h.base, xyzl, h.N * sizeof(double4), hipMemcpyHostToDevice));
     h.mixed = mixed;
     h.L0 = mixed ? 0.0 : L0;
-    return upload_rep(c, r);
+    return set_rep(c, r, c->params[r], h);
 }
 
 int sn_set_lattice_device(sn_ctx *c, int32_t r, const void *xyzl_dev)
@@ -1076,7 +1087,7 @@ int sn_set_lattice_device(sn_ctx *c, int32_t r, const void *xyzl_dev)
     int st = check_rep(c, r);
     if (st) return st;
     if (!xyzl_dev) return fail(c, SN_ERR_INVALID, "null lattice buffer");
-    RepHost &h = c->reps[r];
+    RepHost h = c->reps[r];
     // the caller's writes to xyzl_dev are complete (its streams synchronised);
     // the source is checked before anything is copied, as sn_set_lattice does
     const int nblk = (int)std::min<long long>((h.N + 255) / 256, 1024);
@@ -1092,7 +1103,7 @@ int sn_set_lattice_device(sn_ctx *c, int32_t r, const void *xyzl_dev)
     if (bad > 0.0) return fail(c, SN_ERR_INVALID, "non-finite value in lattice");
     h.mixed = lo != hi;
     h.L0 = h.mixed ? 0.0 : lo;
-    return upload_rep(c, r);
+    return set_rep(c, r, c->params[r], h);
 }
 
 int sn_get_lattice(sn_ctx *c, int32_t r, double *xyzl)
@@ -1134,7 +1145,7 @@ int sn_init_lattice_random(sn_ctx *c, int32_t r, int32_t n_species, const double
         }
         if (acc < 1.0 - 1e-6) return fail(c, SN_ERR_INVALID, "Prevalence must sum to 1");
     }
-    RepHost &h = c->reps[r];
+    RepHost h = c->reps[r];
     // lengths that can occur: species with non-zero prevalence
     std::vector<double> used;
     for (size_t i = 0; i < len.size(); i++)
@@ -1144,13 +1155,14 @@ int sn_init_lattice_random(sn_ctx *c, int32_t r, int32_t n_species, const double
     for (double v : used)
         if (v != used[0]) h.mixed = 1;
     h.L0 = h.mixed ? 0.0 : used[0];
-    if ((st = upload_rep(c, r))) return st;
+    if ((st = check_not_capturing(c))) return st;
     StageLayout lay;
     const size_t o_len = lay.take(len.size() * sizeof(double)), o_cum = lay.take(cum.size() * sizeof(double));
     if ((st = ensure_stage(c, lay.end))) return st;
     double *dl = stage_ptr<double>(c, o_len), *dc = stage_ptr<double>(c, o_cum);
     HIPCHK(c, hipMemcpyAsync(dl, len.data(), len.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(dc, cum.data(), cum.size() * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if ((st = set_rep(c, r, c->params[r], h))) return st;   // (once nothing but the launch can be refused)
     int nblk = (int)((h.N + 255) / 256);
     hipLaunchKernelGGL(init_random_kernel, dim3(nblk), dim3(256), 0, c->stream, c->d_lat, c->d_reps, r,
                        (int)len.size(), dl, dc);
@@ -1164,11 +1176,11 @@ int sn_set_params(sn_ctx *c, int32_t r, double temperature, const double efield[
     int st = check_rep(c, r);
     if (st) return st;
     if (!(temperature >= 0.0)) return fail(c, SN_ERR_INVALID, "temperature must be >= 0");
-    sn_params &p = c->params[r];
+    sn_params p = c->params[r];
     p.temperature = temperature;
     if (efield) { p.efield[0] = efield[0]; p.efield[1] = efield[1]; p.efield[2] = efield[2]; }
     p.cage_strain = cage_strain;
-    return upload_rep(c, r);
+    return set_rep(c, r, p, c->reps[r]);
 }
 
 int sn_site_energy_batch_device(sn_ctx *c, int32_t r, int64_t n, const int32_t *site,

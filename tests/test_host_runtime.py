@@ -87,3 +87,36 @@ before = uploaded.value
 print({call}, uploaded.value > before)           # kept from now on
 """)
     assert out == ["2", "0", "True", "0", "False"]
+
+
+def test_refused_parameters_are_not_kept(run):
+    """Parameters refused under capture reach the device with no later call."""
+    out = run(r"""
+h = context([(12, 12, 12)])
+lat = (D * (4 * 1728))(*([0.0, 0.0, 1.0, 1.0] * 1728))
+def record():                                    # beta, J, L0 of the last parameter record
+    a = bytes(last("put_rep_kernel").arg)
+    return struct.unpack_from("<2d", a, 24) + struct.unpack_from("<d", a, 48)
+capturing.value = 1
+print(L.sn_set_params(h, 0, D(600.0), (D * 3)(0, 0, 0.5), D(7.0)))
+capturing.value = 0
+print(L.sn_set_lattice(h, 0, lat), record() == (1.0, 1.0, 1.0))
+print(L.sn_set_params(h, 0, D(600.0), (D * 3)(0, 0, 0.5), D(7.0)), record() == (0.5, 7.0, 1.0))
+""")
+    assert out == ["2", "0", "True", "0", "True"]
+
+
+@pytest.mark.parametrize("refusal", ["capturing.value = 1", "limit.value = 100"])
+def test_refused_random_lattice_leaves_the_sweep_as_it_was(run, refusal):
+    """A random lattice of several lengths that is refused (capture, no memory
+    for its species table) leaves the kernel variant and the uniform length."""
+    out = run(rf"""
+h = context([(12, 12, 12)])
+print(L.sn_mc_sweeps(h, 1)); before = last("torus_sweep").name
+{refusal}
+print(L.sn_init_lattice_random(h, 0, 2, (D * 2)(0.0, 1.0), (D * 2)(0.5, 0.5)) != 0)
+capturing.value, limit.value = 0, 1 << 40
+print(L.sn_mc_sweeps(h, 1), last("torus_sweep").name == before)
+print(any(b"put_rep" in l.name for l in launches()))
+""")
+    assert out == ["0", "True", "0", "True", "False"]
