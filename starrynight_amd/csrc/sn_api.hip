@@ -179,13 +179,16 @@ static int check_not_capturing(sn_ctx *c)
 
 // Replica r takes parameters p and lattice state h: to the device, in stream
 // order after what is queued, then into the context, which keeps what it had
-// if the launch was refused.
+// if the launch was refused.  (The launch's own status: hipGetLastError would
+// also report what an earlier call of another library left.)
 static int set_rep(sn_ctx *c, int r, const sn_params &p, const RepHost &h)
 {
     int st;
     if ((st = check_not_capturing(c))) return st;
-    hipLaunchKernelGGL(put_rep_kernel, dim3(1), dim3(1), 0, c->stream, c->d_reps + r, make_repdev(p, h));
-    HIPCHK(c, hipGetLastError());
+    RepDev *dst = c->d_reps + r;
+    RepDev rep = make_repdev(p, h);
+    void *args[] = {&dst, &rep};
+    HIPCHK(c, hipLaunchKernel((const void *)put_rep_kernel, dim3(1), dim3(1), args, 0, c->stream));
     c->params[r] = p;
     c->reps[r] = h;
     return SN_OK;

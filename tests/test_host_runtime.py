@@ -120,3 +120,13 @@ print(L.sn_mc_sweeps(h, 1), last("torus_sweep").name == before)
 print(any(b"put_rep" in l.name for l in launches()))
 """)
     assert out == ["0", "True", "0", "True", "False"]
+
+
+def test_parameters_are_not_refused_for_an_earlier_error(run):
+    """An error another library left behind is not this call's."""
+    out = run(r"""
+h = context([(12, 12, 12)])
+C.c_int.in_dll(si, "si_last_error").value = 1
+print(L.sn_set_params(h, 0, D(600.0), None, D(7.0)))
+""")
+    assert out == ["0"]
