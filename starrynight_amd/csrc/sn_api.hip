@@ -37,6 +37,13 @@ struct EnergyList {
     std::vector<char> wide;          // per replica: energy_wide successive x per workgroup, else one
 };
 
+// One round of a whole-lattice sweep: n sites from the colour order's `first`,
+// the first with proposal slot `slot`; a colour's last round ends with the barrier.
+struct TorusRound {
+    int first, n, slot;
+    bool last;
+};
+
 }  // namespace
 
 // Partial sums of sn_gradient_all_device_noalloc: a fixed device array, one
@@ -114,6 +121,9 @@ struct sn_ctx {
     int *d_torus_near[2] = {nullptr, nullptr};
     int torus_max_chunks = 0;
     bool torus_two = false;   // two sites per group and round
+    // what the round tables are made of: a replica of each box size, its rounds
+    std::vector<std::vector<TorusRound>> torus_rounds;
+    std::vector<int> torus_box_rep;
     unsigned long long *d_rep_counters = nullptr;   // 2 per replica (torus sweeps)
     bool can_sweep = false;
     std::string sweep_err;
@@ -137,6 +147,8 @@ static int fail(sn_ctx *c, int code, const std::string &msg)
         if (e_ != hipSuccess)                                                               \
             return fail(ctx, SN_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
+
+static int torus_tables(sn_ctx *c, bool mixed);
 
 static bool any_mixed(const sn_ctx *c)
 {
@@ -191,7 +203,7 @@ static int set_rep(sn_ctx *c, int r, const sn_params &p, const RepHost &h)
     HIPCHK(c, hipLaunchKernel((const void *)put_rep_kernel, dim3(1), dim3(1), args, 0, c->stream));
     c->params[r] = p;
     c->reps[r] = h;
-    return SN_OK;
+    return c->torus && h.mixed ? torus_tables(c, true) : SN_OK;
 }
 
 static void free_graph(sn_ctx *c)
@@ -509,6 +521,59 @@ static long long torus_cost(const std::vector<std::vector<int32_t>> &cstart, int
     return cost;
 }
 
+// The round tables of one LDS layout: own component, proposal slot and
+// neighbours of every lane, 8 + 8 NPL bytes each (sn_torus.h).  Uniform
+// lengths: with the context; mixed: with the first such lattice, since a
+// context seldom needs both.  Neighbours by one table of wrapped coordinates
+// per axis: a 16^3 context at DipoleCutOff 3 takes 2.0 ms, 9.1 ms with both
+// layouts and three wraps a neighbour (0.9 ms are the colouring and the rest).
+static int torus_tables(sn_ctx *c, bool mixed)
+{
+    if (c->d_torus_own[mixed] && c->d_torus_near[mixed]) return SN_OK;
+    const int G = c->torus_G, NPL = c->torus_NPL, rc = c->rc;
+    const int per_round = (c->torus_two ? 2 : 1) * (c->torus_blk / G);
+    size_t sites = 0;   // of all rounds, idle groups' too
+    for (const auto &rounds : c->torus_rounds) sites += rounds.size() * per_round;
+    std::vector<Offset> pairs = neighbour_pairs(rc, c->two_d);
+    pairs.resize(G * NPL, Offset{0, 0, 0, 0});   // a padded pair: the site itself, with no weight
+    std::vector<int2> own(sites * G);
+    std::vector<int> near(sites * G * 2 * NPL);
+    const int prop0 = torus_site_bytes(c, mixed);
+    int2 *o = own.data();
+    int *n = near.data();
+    for (size_t k = 0; k < c->torus_rounds.size(); k++) {
+        const ReplicaGeom &g = c->geom[c->torus_box_rep[k]];
+        const std::vector<int32_t> &order = c->torus_order[c->torus_box_rep[k]];
+        std::vector<int> address((size_t)g.X * g.Y * g.Z), wrap[3];
+        for (size_t i = 0; i < address.size(); i++) address[i] = torus_address((int)i, mixed);
+        const int axis[3] = {g.X, g.Y, g.Z}, stride[3] = {g.Y * g.Z, g.Z, 1};
+        for (int a = 0; a < 3; a++)
+            for (int v = -rc; v < axis[a] + rc; v++) wrap[a].push_back((v + rc * axis[a]) % axis[a] * stride[a]);
+        for (const TorusRound &rd : c->torus_rounds[k])
+            for (int q = 0; q < per_round; q++) {
+                const bool idle = q >= rd.n;
+                const int si = order[idle ? 0 : rd.first + q], slot = idle ? 0 : rd.slot + q;
+                const int *wz = &wrap[2][rc + si % g.Z], *wy = &wrap[1][rc + si / g.Z % g.Y],
+                          *wx = &wrap[0][rc + si / (g.Z * g.Y)];
+                const int flags = (rd.last ? kLast : 0) | (idle ? kIdle : 0);
+                for (int part = 0; part < G; part++) {
+                    *o++ = int2{(address[si] + torus_component(part & 3, mixed)) | flags,
+                                prop0 + 32 * slot + 8 * (part & 3)};
+                    for (int m = 0; m < NPL; m++) {
+                        const Offset &d = pairs[part + m * G];
+                        *n++ = address[wx[d.dx] + wy[d.dy] + wz[d.dz]];
+                        *n++ = address[wx[-d.dx] + wy[-d.dy] + wz[-d.dz]];
+                    }
+                }
+            }
+    }
+    int st;
+    if (!c->d_torus_own[mixed] &&
+        (st = upload_table(c, (void **)&c->d_torus_own[mixed], own.data(), own.size() * sizeof(int2))))
+        return st;
+    return upload_table(c, (void **)&c->d_torus_near[mixed], near.data(), near.size() * sizeof(int));
+}
+
 static int setup_torus(sn_ctx *c)
 {
     const int np = c->npairs;
@@ -585,17 +650,16 @@ static int setup_torus(sn_ctx *c)
     // for (at most the largest replica, at least the largest colour)
     const long long room = (150LL * 1024 / (long long)sizeof(double) - 4LL * c->torus_ms - c->torus_ms / 2) / 4;
     c->torus_pc = (int)std::max<long long>(c->torus_mc, std::min<long long>(room, c->torus_ms));
-    // tables of each box size: the sites by colour, the rounds' entries and
-    // neighbours, the runs of colours whose proposals are drawn together
+    // tables of each box size: the sites by colour, the rounds, the runs of
+    // colours whose proposals are drawn together
     const int NG = blk / G;
     // two sites per group and round where a colour has more sites than the
     // workgroup has groups (and an instance holds them)
     c->torus_two = c->torus_mc > NG && pick_torus(G, NPL, false, blk, true);
     const int R = c->torus_two ? 2 : 1;
-    const std::vector<Offset> pairs = neighbour_pairs(c->rc, c->two_d);
     std::vector<TorusBox> boxes;
-    std::vector<int> box_of, sites, chunks, near[2];
-    std::vector<int2> own[2];
+    std::vector<int> box_of, sites, chunks;
+    long long lane_records = 0;
     std::map<std::array<int, 3>, int> known;
     for (int r = 0; r < c->R; r++) {
         const ReplicaGeom &g = c->geom[r];
@@ -606,7 +670,8 @@ static int setup_torus(sn_ctx *c)
         TorusBox b{};
         b.sites_off = (int)sites.size();
         b.chunk_off = (int)chunks.size();
-        b.round_off = (long long)own[0].size();
+        b.round_off = lane_records;
+        std::vector<TorusRound> rounds;
         sites.insert(sites.end(), o.begin(), o.end());
         const int ncol = (int)cst.size() - 1;
         int p0 = 0;   // first site of the run of colours
@@ -617,40 +682,16 @@ static int setup_torus(sn_ctx *c)
                 chunks.push_back(p0);
                 b.nchunks++;
             }
-            for (int b0 = cst[k]; b0 < cst[k + 1]; b0 += R * NG, b.nrounds++) {
-                const bool last = b0 + R * NG >= cst[k + 1];
-                for (int q = 0; q < R * NG; q++) {
-                    const bool idle = b0 + q >= cst[k + 1];
-                    const int si = idle ? o[0] : o[b0 + q], slot = idle ? 0 : b0 + q - p0;
-                    const int z = si % g.Z, y = si / g.Z % g.Y, x = si / (g.Z * g.Y);
-                    auto wrapped = [&](int a, int bb, int cc) {   // (|offset| < axis)
-                        a += a < 0 ? g.X : a >= g.X ? -g.X : 0;
-                        bb += bb < 0 ? g.Y : bb >= g.Y ? -g.Y : 0;
-                        cc += cc < 0 ? g.Z : cc >= g.Z ? -g.Z : 0;
-                        return (a * g.Y + bb) * g.Z + cc;
-                    };
-                    for (int part = 0; part < G; part++) {
-                        for (int mixed = 0; mixed < 2; mixed++)
-                            own[mixed].push_back(int2{(torus_address(si, mixed) + torus_component(part & 3, mixed)) |
-                                                          (last ? kLast : 0) | (idle ? kIdle : 0),
-                                                      torus_site_bytes(c, mixed) + 32 * slot + 8 * (part & 3)});
-                        for (int m = 0; m < NPL; m++) {
-                            Offset d{0, 0, 0, 0};   // a padded pair: the site itself, with no weight
-                            if (part + m * G < np) d = pairs[part + m * G];
-                            const int sa = wrapped(x + d.dx, y + d.dy, z + d.dz), sb = wrapped(x - d.dx, y - d.dy, z - d.dz);
-                            for (int mixed = 0; mixed < 2; mixed++) {
-                                near[mixed].push_back(torus_address(sa, mixed));
-                                near[mixed].push_back(torus_address(sb, mixed));
-                            }
-                        }
-                    }
-                }
-            }
+            for (int b0 = cst[k]; b0 < cst[k + 1]; b0 += R * NG, b.nrounds++)
+                rounds.push_back(TorusRound{b0, std::min(R * NG, cst[k + 1] - b0), b0 - p0, b0 + R * NG >= cst[k + 1]});
         }
         chunks.push_back(b.nrounds);
         chunks.push_back(cst[ncol]);
         c->torus_max_chunks = std::max(c->torus_max_chunks, b.nchunks);
         boxes.push_back(b);
+        lane_records += (long long)b.nrounds * R * blk;
+        c->torus_box_rep.push_back(r);
+        c->torus_rounds.push_back(rounds);
     }
     // (four arrays, proposals and an int per site: what a replica may take)
     if ((size_t)4 * (c->torus_ms + c->torus_pc) * sizeof(double) + (size_t)c->torus_ms * sizeof(int) > 150 * 1024)
@@ -665,11 +706,8 @@ static int setup_torus(sn_ctx *c)
     if ((st = upload(c, &c->d_torus_box_of, box_of))) return st;
     if ((st = upload(c, &c->d_torus_boxes, boxes))) return st;
     if ((st = upload(c, &c->d_torus_sites, sites))) return st;
-    for (int m = 0; m < 2; m++) {
-        if ((st = upload(c, &c->d_torus_own[m], own[m]))) return st;
-        if ((st = upload(c, &c->d_torus_near[m], near[m]))) return st;
-    }
     if ((st = upload(c, &c->d_torus_chunks, chunks))) return st;
+    if ((st = torus_tables(c, false))) return st;
     std::vector<unsigned long long> z(2 * c->R, 0ull);
     if ((st = upload(c, &c->d_rep_counters, z))) return st;
     c->torus = true;
@@ -1298,6 +1336,7 @@ static int event_pair(sn_ctx *c, std::vector<hipEvent_t> *events, hipEvent_t *e0
 static int launch_torus(sn_ctx *c, int nsw, std::vector<hipEvent_t> *events)
 {
     const bool mixed = any_mixed(c);
+    if (int st = torus_tables(c, mixed)) return st;   // (there, unless an allocation failed)
     TorusArgs t;
     t.lat = c->d_lat; t.reps = c->d_reps; t.pairs = c->d_pairs;
     t.box_of = c->d_torus_box_of; t.boxes = c->d_torus_boxes; t.sites = c->d_torus_sites;

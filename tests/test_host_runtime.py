@@ -130,3 +130,28 @@ C.c_int.in_dll(si, "si_last_error").value = 1
 print(L.sn_set_params(h, 0, D(600.0), None, D(7.0)))
 """)
     assert out == ["0"]
+
+
+def test_round_tables_are_made_for_one_layout_at_a_time(run):
+    """A whole-lattice context makes the round tables of uniform lengths (8 + 8
+    NPL bytes a lane and round, 16^3 at DipoleCutOff 3: about 3.2 MB) and those
+    of mixed lengths with its first such lattice, again after a failure."""
+    out = run(r"""
+h = context([(16, 16, 16)])
+n = 16 ** 3
+at_create = uploaded.value
+lat = (D * (4 * n))(*([0.0, 0.0, 1.0, 1.0] * (n - 1) + [0.0, 1.0, 0.0, 0.0]))
+def tables(call):                                # bytes copied beyond the lattice itself
+    before = uploaded.value
+    return call(), uploaded.value - before - (32 * n if call is set_lattice else 0)
+set_lattice, sweep = lambda: L.sn_set_lattice(h, 0, lat), lambda: L.sn_mc_sweeps(h, 1)
+limit.value = 100000
+print(*[v for call in (set_lattice, sweep) for v in tables(call)])       # refused, and the sweep with it
+limit.value = 1 << 40
+first = tables(sweep)
+print(first[0], 0.9 * at_create < first[1] < at_create < 3.5e6)
+print(*[v for call in (sweep, set_lattice, sweep) for v in tables(call)])
+h = context([(16, 16, 16)])
+print(*[tables(set_lattice) == (0, first[1]), tables(sweep) == (0, 0)])
+""")
+    assert out == ["2", "0", "2", "0", "0", "True", "0", "0", "0", "0", "0", "0", "True", "True"]
