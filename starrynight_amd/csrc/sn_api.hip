@@ -701,6 +701,12 @@ static int setup_torus(sn_ctx *c)
     for (int m = 0; m < 2; m++) {
         const void *f = (const void *)pick_torus(G, NPL, m == 1, blk, c->torus_two);
         if (!f) return fail(c, SN_ERR_UNSUPPORTED, "whole-lattice sweep: no kernel for this cutoff");
+        // the tables hold LDS addresses counted from 0: nothing static may lie before the sites
+        hipFuncAttributes a{};
+        HIPCHK(c, hipFuncGetAttributes(&a, f));
+        if (a.sharedSizeBytes != 0)
+            return fail(c, SN_ERR_HIP, "whole-lattice sweep: the kernel has " + std::to_string(a.sharedSizeBytes) +
+                                           " bytes of static LDS before its sites");
         HIPCHK(c, hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)torus_lds(c, true)));
     }
     if ((st = upload(c, &c->d_torus_box_of, box_of))) return st;

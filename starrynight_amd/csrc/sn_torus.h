@@ -68,8 +68,9 @@ __host__ __device__ inline int torus_component(int c, bool mixed)
     return mixed ? (c >> 1) * 4112 + (c & 1) * 8 : (c < 3 ? c : 2) * 2056;
 }
 
-// LDS at a byte address: the kernel has no static LDS, so its dynamic array,
-// and with it torus_address, begins at 0.  (Through a pointer into the array
+// LDS at a byte address: the kernel has no static LDS (the host refuses an
+// instance that has any), so its dynamic array, and with it torus_address,
+// begins at 0.  (Through a pointer into the array
 // every read of a table's address cost an add of that zero.)
 typedef double lds_double2 __attribute__((ext_vector_type(2)));
 template <typename T>

@@ -14,6 +14,7 @@ size_t si_uploaded;                /* bytes copied host to device */
 int si_copy_fails;                 /* synchronous copies fail */
 int si_capturing;                  /* every stream is under capture */
 int si_last_error;                 /* what hipGetLastError returns */
+size_t si_static_lds;              /* static LDS of every kernel */
 
 /* ---- launches ---- */
 enum { MAX_KERNELS = 4096, KEEP = 64 };
@@ -107,6 +108,12 @@ int hipGetDevice(int *d) { *d = 0; return OK; }
 int hipDeviceGetAttribute(int *v, int attribute, int device) { (void)attribute; (void)device; *v = 256; return OK; }
 int hipGetDevicePropertiesR0600(void *p, int device) { (void)p; (void)device; return INVALID_VALUE; }
 int hipFuncSetAttribute(const void *f, int attribute, int value) { (void)f; (void)attribute; (void)value; return OK; }
+int hipFuncGetAttributes(void *a, const void *f)
+{
+    (void)f;
+    memcpy((char *)a + 48, &si_static_lds, sizeof si_static_lds); /* sharedSizeBytes */
+    return OK;
+}
 const char *hipGetErrorString(int e) { return e == OUT_OF_MEMORY ? "out of memory" : "error"; }
 int hipGetLastError(void) { int e = si_last_error; si_last_error = 0; return e; }
 int hipStreamCreateWithFlags(void **s, unsigned flags) { (void)flags; *s = &handle; return OK; }

@@ -155,3 +155,16 @@ h = context([(16, 16, 16)])
 print(*[tables(set_lattice) == (0, first[1]), tables(sweep) == (0, 0)])
 """)
     assert out == ["2", "0", "2", "0", "0", "True", "0", "0", "0", "0", "0", "0", "True", "True"]
+
+
+def test_whole_lattice_kernel_with_static_lds_is_refused(run):
+    """Its tables hold LDS addresses that begin at 0: an instance whose sites
+    would begin elsewhere is not launched."""
+    out = run(r"""
+print(create([(25, 25, 1)])[0], create([(25, 25, 1)], kernel=3)[0])
+C.c_size_t.in_dll(si, "si_static_lds").value = 16
+for kernel in (0, 3):
+    status, h = create([(25, 25, 1)], kernel=kernel)
+    print(status, b"static LDS" in L.sn_last_error(h))
+""")
+    assert out == ["0", "0", "2", "True", "2", "True"]
