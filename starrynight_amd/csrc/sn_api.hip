@@ -85,7 +85,7 @@ struct sn_ctx {
     void *d_radial = nullptr;         // radial-order columns, bin starts and entries (built on first use)
     size_t radial_start = 0, radial_entries = 0;   // byte offsets of the last two
     std::vector<int> radial_count;    // offsets per bin
-    int cus = 0;                      // compute units of the device (set with the radial tables)
+    int cus = 0;                      // compute units of the device
     double *d_stencil[kFieldMaxR + 1] = {};   // weights: 0 potential, c > 0 field of cutoff c (built on first use)
     double *d_obs = nullptr;          // observable output staging
     size_t obs_cap = 0;
@@ -273,7 +273,6 @@ static int energy_list(sn_ctx *c, bool together, EnergyList &list)
     const int nx_wide = energy_wide(c->rc, c->two_d), rc = c->rc;
     struct Split { int zl, nz, valid, ny, rows; };
     std::vector<Split> split(c->R);
-    constexpr int kCUs = 256;
     for (int r = 0; r < c->R; r++) {
         const RepHost &h = c->reps[r];
         // the cut of a row into nz (1: whole, no halo) that leaves the fewest
@@ -306,7 +305,7 @@ static int energy_list(sn_ctx *c, bool together, EnergyList &list)
                 long long blocks = 0;
                 for (int r = r0; r < r1; r++)
                     blocks += (long long)((c->reps[r].X + step * steps - 1) / (step * steps)) * split[r].ny * split[r].nz;
-                const double cost = (double)((blocks + kCUs - 1) / kCUs) * (steps * (2 * rc + 2 * step) + 6);
+                const double cost = (double)((blocks + c->cus - 1) / c->cus) * (steps * (2 * rc + 2 * step) + 6);
                 if (best < 0.0 || cost < best) { best = cost; nx = step; len = step * steps; }
             }
     };
@@ -378,9 +377,9 @@ static void launch_reduce(sn_ctx *c, int nblk, int width)
 constexpr int kMaxRegion = 4096;
 // Replicas of at most this many sites sweep with the whole-lattice kernel
 // when the tuning leaves the kernel to the library (and it fits in LDS).
-// Measured against gather tiles, site-updates/s at DipoleCutOff 3: 14^3
-// +40-44%, 16 x 16 x 12 +80%, 16^3 +0-6% (one or 64 replicas); 16^3 at
-// DipoleCutOff 4 +21-25% (5-10% half vacant), at 3 half vacant -7-10%.
+// Measured against gather tiles at DipoleCutOff 3, one replica and 64: 12^3
+// 3.0-3.1x, 14^3 2.0-2.1x, 16 x 16 x 12 2.4x, 16^3 +12-17% (half vacant
+// +4-8%); 16^3 at DipoleCutOff 4 +46-51% (half vacant -11-17%).
 constexpr long long kAutoTorusSites = 4096;
 // Largest tile: the field kernel gives each lane at most 2 items of 2 sites
 // (3D) or 1 site (2D).
@@ -905,6 +904,7 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
                                                std::to_string(max_class) + " sites)");
 
     HIPCHK(c, hipGetDevice(&c->device));
+    HIPCHK(c, hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
     if (int se = resolve_scratch(c)) return se;
     HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     HIPCHK(c, hipMalloc((void **)&c->d_lat, (size_t)c->total_sites * sizeof(double4)));
@@ -1294,7 +1294,7 @@ static SweepArgs sweep_args(sn_ctx *c)
     a.sites = c->d_sites; a.gsteps = c->d_gsteps;
     a.prop_stride = c->prop_chunk;
     a.pairs = c->d_pairs; a.sweep_ctr = c->d_sweep; a.counters = c->d_counters;
-    a.npairs = c->npairs; a.rc = c->rc; a.two_d = c->two_d ? 1 : 0;
+    a.rc = c->rc; a.two_d = c->two_d ? 1 : 0;
     a.max_region = c->gather_region;
     return a;
 }
@@ -1618,7 +1618,9 @@ static int run_energy(sn_ctx *c, int r, double *dg, double *fixed_partials = nul
     };
     double *part = nullptr;
     if (c->energy_rows) {
-        if (fixed_partials) {   // a row per tile, or per 256 sites of the largest replica without tiles
+        // the bound that the entry point states: a row per tile, or per 256
+        // sites of the largest replica without tiles (the kernel needs fewer)
+        if (fixed_partials) {
             long long rows = 0;
             for (int q = all ? 0 : r; q < (all ? c->R : r + 1); q++)
                 rows = c->scratch_rows.empty() ? std::max(rows, (c->reps[q].N + 255) / 256) : rows + c->scratch_rows[q];
@@ -1805,7 +1807,6 @@ static int ensure_radial(sn_ctx *c)
     start[kRadialBins] = (int)entries.size();
     HIPCHK(c, hipFuncSetAttribute((const void *)radial_order_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   kRadialLds));
-    HIPCHK(c, hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device));
     // one allocation: columns, bin starts, entries
     const size_t at_start = cols.size() * sizeof(RadialCol), at_entries = at_start + start.size() * sizeof(int);
     std::vector<char> table(at_entries + entries.size() * sizeof(unsigned short));

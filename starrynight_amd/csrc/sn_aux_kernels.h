@@ -21,11 +21,10 @@ struct FieldOut {
 };
 
 __device__ __forceinline__ void site_field(const double4 *lat, const RepDev &rep, const PairDev *offs,
-                                           int noff, int x, int y, int z, int first, int stride,
-                                           FieldOut &f)
+                                           int noff, int x, int y, int z, FieldOut &f)
 {
     f.hx = f.hy = f.hz = f.gx = f.gy = f.gz = 0.0;
-    for (int i = first; i < noff; i += stride) {
+    for (int i = 0; i < noff; i++) {
         const PairDev o = offs[i];
         int gx = wrap_once(x + o.dx, rep.X), gy = wrap_once(y + o.dy, rep.Y), gz = wrap_once(z + o.dz, rep.Z);
         double4 t = lat[((long long)gx * rep.Y + gy) * rep.Z + gz];
@@ -272,7 +271,7 @@ __global__ __launch_bounds__(256) void energy_grad_kernel(const double4 *lat, co
         int z = (int)(s % rep.Z), q = (int)(s / rep.Z), y = q % rep.Y, x = q / rep.Y;
         double4 p = L[s];
         FieldOut f;
-        site_field(L, rep, offs, noff, x, y, z, 0, 1, f);
+        site_field(L, rep, offs, noff, x, y, z, f);
         double ph = p.x * f.hx + p.y * f.hy + p.z * f.hz;
         double pg = p.x * f.gx + p.y * f.gy + p.z * f.gz;
         double gx = p.w * f.hx - rep.J * f.gx + rep.E[0];

@@ -19,13 +19,12 @@ struct SweepArgs {
     const RepDev *reps;
     const TileDev *tiles;
     const ShapeDev *shapes;
-    const PairDev *pairs;
+    const PairDev *pairs;      // padded with zero pairs to kPairSlots
     const unsigned *sweep_ctr;
     unsigned long long *counters;  // 2 per tile: accepted, rejected (accumulated over sweeps)
     const int *sites;         // per shape (TileDev.sites_off): tile sites by fine colour, packed lx | ly << 10 | lz << 20
     const int *gsteps;        // per shape (TileDev.gstep_off): per step BLK / G entries (step_entry), an idle row, then
                               // the first step and the first site of each proposal chunk (nchunks + 1 of both)
-    int npairs;               // (the table is padded with zero pairs to kPairSlots)
     int rc, two_d, max_region;
     int prop_stride;          // proposal slots per chunk (<= kBlock)
 };

@@ -8,7 +8,7 @@
 // through the periodic boundary and update together; colours follow one
 // another with a workgroup barrier.  The neighbours' LDS addresses (periodic
 // wrap, the reference's % X, src/starrynight-montecarlo-core.c:97) come from a
-// table of the replica's box, streamed from L2 two rounds ahead: forming them in
+// table of the replica's box, streamed from L2 three rounds ahead: forming them in
 // the round took 66 of its instructions (25 x 25), after the barrier.
 // Per site the arithmetic is the tile kernels': G lanes share a site, each
 // lane takes NPL of the +-r pairs, one scalar per lane is reduced over the
@@ -86,7 +86,7 @@ __device__ __forceinline__ void lds_store(int address, double v)
 // R sites per group and round, of one colour: with one (colours that fit the
 // groups) a round's latencies follow one another; two sites' reads, sums and
 // reductions overlap (64 x 12^3 at DipoleCutOff 3, 54 sites a colour on 16
-// groups, 10 sweeps: 710 -> 641 us).
+// groups, 10 sweeps: 643 -> 569 us).
 template <int G, int NPL, bool MIXED, int BLK, int R>
 __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nsweeps)
 {
@@ -230,8 +230,8 @@ __global__ __launch_bounds__(BLK) void torus_sweep_kernel(TorusArgs t, int nswee
                         }
                     };
                     // two sites: reads run two pairs ahead of the sums (see the
-                    // tile sweep; 64 x 12^3, 10 sweeps: 641 us, all reads
-                    // first 702)
+                    // tile sweep; 64 x 12^3, 10 sweeps: 565 us, all reads
+                    // first 617)
                     constexpr int AHEAD = R == 1 || R * NPL < 2 ? R * NPL : 2;
 #pragma unroll
                     for (int k = 0; k < AHEAD; k++) pair_reads(k / NPL, k % NPL);
