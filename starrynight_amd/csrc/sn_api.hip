@@ -390,8 +390,8 @@ static bool plan(const std::vector<ReplicaGeom> &geom, int rc, const sn_tuning &
 {
     // default edge targets: 8^3 in 3D (the 14^3 staged region at rc = 3);
     // 16 x 16 in 2D, where a tile's region stays small and its colour classes
-    // grow from about 6 to 26 sites (1024^2 at rc = 3: 1.03e10 site-updates/s
-    // against 5.5e9 with 8 x 8 tiles; rc = 4: 6.8e9 against 4.8e9)
+    // grow from about 6 to 26 sites (1024^2 at rc = 3: 1.45e10 site-updates/s
+    // against 7.0e9 with 8 x 8 tiles; rc = 4: 8.6e9 against 5.7e9)
     const bool two_d = geom[0].Z == 1;
     const int d = two_d ? 16 : 8;
     int target[3] = {t.tile[0] > 0 ? t.tile[0] : d, t.tile[1] > 0 ? t.tile[1] : d,
@@ -492,8 +492,8 @@ static size_t torus_lds(const sn_ctx *c, bool mixed)
 // lanes per site, pairs per lane and threads for npairs pairs and colours of
 // at most mc sites: 1024 threads when a colour has enough sites to keep them
 // busy.  The greedy colourings' colours of up to 64 sites (wide) take 8 lanes
-// x 2 pairs in 512 threads (measured at 25 x 25: 4.3e7 site-updates/s against
-// 4.1e7 with 16 lanes in 1024 threads).
+// x 2 pairs in 512 threads (measured at 25 x 25 against 16 lanes in 1024
+// threads: 7.9e7 to 7.8e7 site-updates/s, 512 replicas 2.75e10 to 1.95e10).
 static bool torus_shape(int np, int mc, bool wide, int &G, int &NPL, int &blk)
 {
     blk = 256;
@@ -815,10 +815,10 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     if (blk != 256 && blk != 512) return fail(c, SN_ERR_INVALID, "block_threads must be 256 or 512");
     if (c->tuning.kernel < 0 || c->tuning.kernel > 3) return fail(c, SN_ERR_INVALID, "kernel must be 0..3");
     // kernel 0 picks by size (rates measured on MI355X): the whole-lattice
-    // kernel for replicas of up to kAutoTorusSites sites (2-3x the gather
-    // kernel at 12^3 and 25x25), else the per-phase gather kernel (1.2-2x the
+    // kernel for replicas of up to kAutoTorusSites sites (3-5x the gather
+    // kernel at 12^3 and 25x25), else the per-phase gather kernel (1.5-2.3x the
     // field-update kernel from 16^3 to 128^3 at DipoleCutOff 2-4, batched or
-    // not; 2.3-2.6x at DipoleCutOff 1 and 1.55x at 5, 64^3 and 128^3), else
+    // not; 2.4-3.1x at DipoleCutOff 1 and 1.7-1.8x at 5, 64^3 and 128^3), else
     // the field-update kernel where no gather instance fits
     int kern = c->tuning.kernel;
     if (kern == 0 && blk != kBlock) kern = 2;
@@ -837,9 +837,9 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     // Lanes per site: the G whose groups hold a colour class in one step
     // (down to 4 lanes) with the fewest pair slots G x NPL, the larger G on
     // a tie.  Measured at 1024^2 (2D), site-updates/s: DipoleCutOff 3 (14
-    // pairs) 16 x 1 5.8e9 against 32 x 2 4.7e9; DipoleCutOff 4 (24 pairs)
-    // 16 x 2 4.8e9 against 32 x 2 4.3e9; DipoleCutOff 2 (6 pairs) 4 x 2
-    // 6.8e9 against 16 x 1 6.7e9.  3D lattices keep 16 x 4 (61 pairs) and
+    // pairs) 1.46e10 against 1.36e10 with 16 lanes and 7.9e9 with 32;
+    // DipoleCutOff 4 (24 pairs) 8.6e9 against 7.2e9 with 32; DipoleCutOff 2
+    // (6 pairs) 1.54e10 against 1.28e10 with 16.  3D lattices keep 16 x 4 (61 pairs) and
     // 16 x 8 (128), and DipoleCutOff 5 (257 pairs) takes 64 x 5.
     auto lane_shape = [&](int threads, int &G, int &NPL) {
         G = c->tuning.lanes_per_site;
@@ -865,14 +865,14 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     lane_shape(blk, G, NPL);
     // The gather kernel runs 512 threads, unless the tuning fixes the block
     // or the lanes, where 256 threads at 4 lanes a site hold fewer sites than
-    // a colour class (DipoleCutOff 1: 4 lanes x 1 pair, 1.06-1.09x the
-    // 256-thread rate at 64^3 and 128^3).  DipoleCutOff 5 stays at 256
-    // threads, 64 lanes x 5 pairs: 1.16x 512 threads of 64 lanes x 8 pairs,
-    // 1.55x the field-update kernel at 128^3.
+    // a colour class (DipoleCutOff 1: 4 lanes x 1 pair, 1.07x the 256-thread
+    // rate at 64^3, the same at 128^3).  DipoleCutOff 5 stays at 256
+    // threads, 64 lanes x 5 pairs: 1.34x 512 threads of 64 lanes x 8 pairs,
+    // 1.7x the field-update kernel at 128^3.
     // It also runs 512 threads where its staged region leaves room for one
     // 256-thread workgroup per CU (four waves) and 512 threads give a site
     // twice the lanes: 128^3 at DipoleCutOff 4 (16^3 region), 32 lanes x 4
-    // pairs against 16 x 8, +4% (+17% half vacant).
+    // pairs against 16 x 8, +1% (+19% half vacant).
     int region = 0;
     for (const TileShape &s : c->sched.shapes)
         region = std::max(region, (s.tx + 2 * c->rc) * (s.ty + 2 * c->rc) *
