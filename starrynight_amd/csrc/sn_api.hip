@@ -1294,7 +1294,7 @@ static SweepArgs sweep_args(sn_ctx *c)
     a.sites = c->d_sites; a.gsteps = c->d_gsteps;
     a.prop_stride = c->prop_chunk;
     a.pairs = c->d_pairs; a.sweep_ctr = c->d_sweep; a.counters = c->d_counters;
-    a.rc = c->rc; a.two_d = c->two_d ? 1 : 0;
+    a.npairs = c->npairs; a.rc = c->rc; a.two_d = c->two_d ? 1 : 0;
     a.max_region = c->gather_region;
     return a;
 }

@@ -25,6 +25,8 @@ struct SweepArgs {
     const int *sites;         // per shape (TileDev.sites_off): tile sites by fine colour, packed lx | ly << 10 | lz << 20
     const int *gsteps;        // per shape (TileDev.gstep_off): per step BLK / G entries (step_entry), an idle row, then
                               // the first step and the first site of each proposal chunk (nchunks + 1 of both)
+    int npairs;               // read by no kernel, but the arguments behind it stay where they are: without it tiles
+                              // of mixed lengths ran 2% faster, some of uniform lengths 1% slower
     int rc, two_d, max_region;
     int prop_stride;          // proposal slots per chunk (<= kBlock)
 };
