@@ -379,7 +379,7 @@ constexpr int kMaxRegion = 4096;
 // when the tuning leaves the kernel to the library (and it fits in LDS).
 // Measured against gather tiles at DipoleCutOff 3, one replica and 64: 12^3
 // 3.0-3.1x, 14^3 2.0-2.1x, 16 x 16 x 12 2.4x, 16^3 +12-17% (half vacant
-// +4-8%); 16^3 at DipoleCutOff 4 +46-51% (half vacant -11-17%).
+// +4-8%); 16^3 at DipoleCutOff 4 +43-49% (half vacant -9-14%).
 constexpr long long kAutoTorusSites = 4096;
 // Largest tile: the field kernel gives each lane at most 2 items of 2 sites
 // (3D) or 1 site (2D).
@@ -493,7 +493,7 @@ static size_t torus_lds(const sn_ctx *c, bool mixed)
 // at most mc sites: 1024 threads when a colour has enough sites to keep them
 // busy.  The greedy colourings' colours of up to 64 sites (wide) take 8 lanes
 // x 2 pairs in 512 threads (measured at 25 x 25 against 16 lanes in 1024
-// threads: 7.9e7 to 7.8e7 site-updates/s, 512 replicas 2.75e10 to 1.95e10).
+// threads: 7.8e7 to 7.7e7 site-updates/s, 512 replicas 2.74e10 to 1.95e10).
 static bool torus_shape(int np, int mc, bool wide, int &G, int &NPL, int &blk)
 {
     blk = 256;
@@ -837,9 +837,9 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     // Lanes per site: the G whose groups hold a colour class in one step
     // (down to 4 lanes) with the fewest pair slots G x NPL, the larger G on
     // a tie.  Measured at 1024^2 (2D), site-updates/s: DipoleCutOff 3 (14
-    // pairs) 1.46e10 against 1.36e10 with 16 lanes and 7.9e9 with 32;
+    // pairs) 1.46e10 against 1.35e10 with 16 lanes and 8.0e9 with 32;
     // DipoleCutOff 4 (24 pairs) 8.6e9 against 7.2e9 with 32; DipoleCutOff 2
-    // (6 pairs) 1.54e10 against 1.28e10 with 16.  3D lattices keep 16 x 4 (61 pairs) and
+    // (6 pairs) 1.53e10 against 1.28e10 with 16.  3D lattices keep 16 x 4 (61 pairs) and
     // 16 x 8 (128), and DipoleCutOff 5 (257 pairs) takes 64 x 5.
     auto lane_shape = [&](int threads, int &G, int &NPL) {
         G = c->tuning.lanes_per_site;
@@ -865,14 +865,14 @@ int sn_create(const sn_params *params, int32_t n_replicas, const sn_tuning *tuni
     lane_shape(blk, G, NPL);
     // The gather kernel runs 512 threads, unless the tuning fixes the block
     // or the lanes, where 256 threads at 4 lanes a site hold fewer sites than
-    // a colour class (DipoleCutOff 1: 4 lanes x 1 pair, 1.07x the 256-thread
+    // a colour class (DipoleCutOff 1: 4 lanes x 1 pair, 1.06x the 256-thread
     // rate at 64^3, the same at 128^3).  DipoleCutOff 5 stays at 256
     // threads, 64 lanes x 5 pairs: 1.34x 512 threads of 64 lanes x 8 pairs,
     // 1.7x the field-update kernel at 128^3.
     // It also runs 512 threads where its staged region leaves room for one
     // 256-thread workgroup per CU (four waves) and 512 threads give a site
     // twice the lanes: 128^3 at DipoleCutOff 4 (16^3 region), 32 lanes x 4
-    // pairs against 16 x 8, +1% (+19% half vacant).
+    // pairs against 16 x 8, +4% (+16% half vacant).
     int region = 0;
     for (const TileShape &s : c->sched.shapes)
         region = std::max(region, (s.tx + 2 * c->rc) * (s.ty + 2 * c->rc) *
